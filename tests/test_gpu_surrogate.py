@@ -118,3 +118,17 @@ def test_surrogate_saves_iterations_same_solution(wflib):
     assert s["iters"] / s["calls"] < p["iters"] / p["calls"]
     for k in ["u", "sigma", "pl_strain", "T"]:
         assert rel_l2(s["fields"][k], p["fields"][k]) < 1e-8, k
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 127, 128, 129, 4097, 32768, 32769, 40001])
+def test_mlp_gradient_sample_counts(wflib, n):
+    """Sample counts at the edges of a wavefront's 32, a block's 128 and the
+    256 blocks' 32,768 (FP32 sums against FP64: relative L2 <= 1e-4)."""
+    w, X, Y = _data(100 + n, n)
+    with _dom(wflib) as d:
+        d.set_mlp_params(w)
+        g, loss = d.mlp_grad(X, Y)
+    g_ref, loss_ref = po.mlp_loss_grad(w.astype(np.float64), X.astype(np.float64),
+                                       Y.astype(np.float64))
+    assert rel_l2(g, g_ref) < 1e-4
+    assert abs(loss - loss_ref) < 1e-5 * max(1.0, loss_ref)

@@ -171,7 +171,7 @@ struct StatsFold {
 };
 
 constexpr int kMlpParams = 1249;  // 4x32 + 32 + 32x32 + 32 + 32 + 1
-constexpr int kMlpMaxBlocks = 256;  // gradient blocks (one 64-sample chunk each)
+constexpr int kMlpMaxBlocks = 256;  // gradient blocks (at least one 128-sample chunk each)
 constexpr int kMlpOffW1 = 0, kMlpOffB1 = 128, kMlpOffW2 = 160, kMlpOffB2 = 1184,
               kMlpOffW3 = 1216, kMlpOffB3 = 1248;
 
@@ -324,7 +324,7 @@ void launch_mlp_grad(hipStream_t s, const float* w, const float* X, const float*
 void launch_mlp_train_iter(hipStream_t s, float* w, float* m, float* v, const float* X,
                            const float* Y, int n, int stride, float* part, float* loss_part,
                            int nblocks, int t, float lr, float* loss);
-// gradient blocks for n samples: one 64-sample chunk each, at most kMlpMaxBlocks
+// gradient blocks for n samples: one 128-sample chunk each, at most kMlpMaxBlocks
 int mlp_grad_blocks(int n);
 // record msg as the calling thread's wf_last_error() text; returns code
 int set_last_error(int code, const char* msg);
