@@ -1,0 +1,72 @@
+"""Pair loops with the neighbours staged whole in LDS.
+
+They take domains whose particles share one h, and in the acceleration one
+sound speed (FP64: and one mass); other domains keep the gathering loops and
+the general record.  Both must give the same passes at every tile remainder,
+and a domain that changes from one to the other must not use stale records.
+
+Tolerances: against the FP64 oracle, one call, relative L2 <= 1e-12 (FP64:
+rounding of ~56 terms a sum) and 2e-5 (mixed: FP32 terms).
+"""
+import numpy as np
+import pytest
+
+from weldformgpu_amd import _abi, scenarios
+
+from harness import randomize, rel_l2, to_gpu, to_oracle
+
+pytestmark = pytest.mark.gpu
+
+TOL = {_abi.WF_FP64: 1e-12, _abi.WF_MIXED: 2e-5}
+
+
+def _scenario(n, precision, beta):
+    """The first n particles of a thermo-mechanical cylinder, random v, stress
+    and temperature."""
+    sc = scenarios.c3_johnson_cook(scale=0.2)
+    for k, v in sc.fields.items():
+        sc.fields[k] = v[:n].copy()
+    sc.cfg.n_particles = sc.cfg.solid_count = n
+    sc.cfg.precision = precision
+    sc.cfg.beta = beta
+    randomize(sc, seed=n)
+    rng = np.random.default_rng(n)
+    sc.fields["T"] = 300.0 + rng.uniform(0.0, 50.0, n)
+    sc.fields["k_T"] = rng.choice([150.0, 200.0], n)
+    return sc
+
+
+def _passes(d, st, cfg, tol):
+    d.CalcDensInc()
+    st.calc_dens_inc(cfg)
+    d.CalcRateTensors()
+    st.calc_rate_tensors(cfg)
+    d.CalcAccel()
+    st.calc_accel(cfg)
+    d.CalcTempInc()
+    st.calc_temp_inc(cfg)
+    for k in ("drho", "strrate", "rotrate", "a", "dTdt"):
+        assert rel_l2(d.get(k), st[k]) <= tol, k
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("n", [1, 63, 127, 128, 129, 1000, 4481])
+def test_uniform_and_general_passes(oracle, wflib, n, precision):
+    sc = _scenario(n, precision, 1.0 if n == 129 else 0.0)
+    st = to_oracle(oracle, sc)
+    st.nsearch(sc.cfg)
+    with to_gpu(sc, wflib) as d:
+        d.nsearch()
+        _passes(d, st, sc.cfg, TOL[precision])
+        # one particle apart in Cs, then in m, then in h: the general loops
+        for k, f in (("Cs", 1.01), ("m", 1.01), ("h", 1.0 + 1e-6)):
+            a = st[k].copy()
+            a[n // 2] *= f
+            st[k] = a
+            d.set(k, a)
+            _passes(d, st, sc.cfg, TOL[precision])
+        # and back
+        for k in ("h", "m", "Cs"):
+            st[k] = sc.fields[k]
+            d.set(k, sc.fields[k])
+        _passes(d, st, sc.cfg, TOL[precision])

@@ -133,6 +133,14 @@ struct wf_domain {
   bool uniform_h = true;     // every particle has the same h (FP32 loops skip h_j)
   bool uniform_m = true;     // every particle has the same mass m_value (the
   double m_value = 0.0;      // surface pass skips the neighbour-mass gather)
+  bool uniform_cs = true;    // and the same sound speed cs_value
+  double cs_value = 0.0;
+  // the FP64 acceleration record's layout (Fields::arec64u), after a change
+  // of h, m or Cs; the records are then rewritten before the next pass
+  bool uniform_c() const { return uniform_h && uniform_cs; }
+  void pick_arec64() {
+    f.arec64u = !mixed && uniform_c() && uniform_m ? f.arec64 + npad : nullptr;
+  }
   bool mirror_dirty = true;  // FP32 mirrors out of date with the FP64 state
   bool nb_built = false;
   bool snapshot_set = false;
@@ -744,6 +752,7 @@ int wf_create(const wf_config* cfg, wf_domain** out) {
     for (double4** q : d4)
       if (!rc) rc = d->dev_alloc((void**)q, sizeof(double4) * d->npad);
     if (!rc) rc = d->dev_alloc((void**)&d->f.arec64, 3 * sizeof(double4) * d->npad);
+    d->pick_arec64();
   }
   // return-map statistics, surrogate samples and weights
   d->jc_newton = cfg->return_map == WF_RETURN_NEWTON && cfg->mat.model == WF_MAT_JOHNSON_COOK;
@@ -908,6 +917,13 @@ int wf_set_field(wf_domain* d, int field, const void* host, size_t bytes) {
     d->m_value = mv[0];
     for (int i = 1; i < d->n && d->uniform_m; i++) d->uniform_m = mv[i] == mv[0];
   }
+  if (field == WF_F_CS) {
+    const double* cv = (const double*)host;
+    d->uniform_cs = true;
+    d->cs_value = cv[0];
+    for (int i = 1; i < d->n && d->uniform_cs; i++) d->uniform_cs = cv[i] == cv[0];
+  }
+  d->pick_arec64();
   HIPC(hipMemcpyAsync(d->stage, host, bytes, hipMemcpyHostToDevice, d->stream));
   if (elem == 8 && d->plane(field, 0).f) {
     Planes6f planes{};
@@ -1006,6 +1022,11 @@ int wf_fill_field(wf_domain* d, int field, double value) {
     d->m_value = value;
   }
   if (field == WF_F_H) d->uniform_h = true;
+  if (field == WF_F_CS) {
+    d->uniform_cs = true;
+    d->cs_value = value;
+  }
+  d->pick_arec64();
   if (field == WF_F_X) {
     for (int c = 0; c < 3; c++) launch_fill_f64(d->stream, d->f.xs[c], value, d->n);
     d->snap_gen++;
@@ -1294,10 +1315,10 @@ int wf_calc_accel(wf_domain* d) {
   d->refresh_mirrors();
   if (d->mixed)
     launch_accel_mixed(d->stream, d->f, d->tl, d->solid, d->cfg.alpha, d->cfg.beta,
-                       d->frame.cs32, d->uniform_h);
+                       d->frame.cs32, d->uniform_h, d->uniform_c(), d->cs_value);
   else
     launch_accel_tiled(d->stream, d->f, d->tl, d->solid, d->cfg.alpha, d->cfg.beta,
-                       d->uniform_h);
+                       d->uniform_h, d->m_value, d->cs_value);
   HIPC(hipGetLastError());
   return WF_OK;
 }
@@ -1712,14 +1733,18 @@ int wf_step(wf_domain* d, int n_steps) {
         out.p4 = d->p4_spare;
         out.v4 = d->f.v4_alt;
         launch_accel_integrate_mixed(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, cs32, uh,
-                                     d->cfg.dt, d->bcs, d->frame, out, fold);
+                                     d->uniform_c(), d->cs_value, d->cfg.dt, d->bcs, d->frame,
+                                     out, fold);
         std::swap(d->f.p4, d->p4_spare);
         std::swap(d->f.v4, d->f.v4_alt);
         if ((rc = timer_end(d, WF_K_ACCEL_INTEGRATE))) return rc;
       } else {
         if (mx)
-          launch_accel_mixed(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, cs32, uh, fold);
-        else launch_accel_tiled(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, uh, fold);
+          launch_accel_mixed(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, cs32, uh,
+                             d->uniform_c(), d->cs_value, fold);
+        else
+          launch_accel_tiled(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, uh, d->m_value,
+                             d->cs_value, fold);
         if (d->cfg.axisymm) launch_axisymm_bc(d->stream, d->f, d->n);  // SolverFraser.cu:229-231
         if ((rc = timer_end(d, WF_K_ACCEL))) return rc;
       }
@@ -1979,9 +2004,12 @@ int wf_time_pass(wf_domain* d, int k, int reps, double* ms_per_launch) {
       if (mx) launch_rates_mixed(d->stream, d->f, d->tl, d->solid, d->cfg.quirks, cs32, uh);
       else launch_rates_tiled(d->stream, d->f, d->tl, d->solid, d->cfg.quirks, uh);
     } else {
-      if (mx) launch_accel_mixed(d->stream, d->f, d->tl, d->solid, d->cfg.alpha, d->cfg.beta,
-                                 cs32, uh);
-      else launch_accel_tiled(d->stream, d->f, d->tl, d->solid, d->cfg.alpha, d->cfg.beta, uh);
+      if (mx)
+        launch_accel_mixed(d->stream, d->f, d->tl, d->solid, d->cfg.alpha, d->cfg.beta, cs32, uh,
+                           d->uniform_c(), d->cs_value);
+      else
+        launch_accel_tiled(d->stream, d->f, d->tl, d->solid, d->cfg.alpha, d->cfg.beta, uh,
+                           d->m_value, d->cs_value);
     }
   };
   launch();  // warm

@@ -53,6 +53,11 @@ struct Fields {
   // sigma/rho^2 {xx, yy, zz, xy}, {sigma/rho^2 yz, xz, rho, Cs}, and
   // tk64 = {T, k, m/rho, 0} (double-buffered)
   double4 *kv, *kv_alt, *arec64, *tk64, *tk64_alt;
+  // non-null when every particle has the same h, mass and sound speed: the
+  // acceleration record is then split into what its pass stages in LDS,
+  // arec64u[i] = {sigma/rho^2 xx, yy, rho, 0}, and what a pair gathers,
+  // arec64[i] = sigma/rho^2 {zz, xy, yz, xz} (both in arec64's allocation)
+  double4* arec64u;
   // return-map surrogate training samples, one slot per particle: features
   // (s_trial/A, 10 eps_p, log10(max(rate,1e-3))/3, theta), target dg/dg_max,
   // step of the sample (-1: none)
@@ -254,7 +259,8 @@ void launch_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int 
 void launch_rates_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         int quirks, bool uh);
 void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        double alpha, double beta, bool uh, const StatsFold& fold = {});
+                        double alpha, double beta, bool uh, double m_uni, double cs_uni,
+                        const StatsFold& fold = {});
 void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
                        double h_conv, double dt, bool leap, bool first, bool uh);
 
@@ -263,18 +269,19 @@ void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int 
 // non-axisymmetric steps with every particle solid); the new positions and
 // FP32 mirrors go to out's planes (IntegrateOut, above)
 void launch_accel_integrate_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                                  double alpha, double beta, float cs32, bool uh, double dt,
-                                  const BcTable& bc, const Frame32& fr, const IntegrateOut& out,
-                                  const StatsFold& fold = {});
+                                  double alpha, double beta, float cs32, bool uh, bool uc,
+                                  double cs_uni, double dt, const BcTable& bc, const Frame32& fr,
+                                  const IntegrateOut& out, const StatsFold& fold = {});
 
 // mixed precision (FP32 pair loops, FP32 terms summed in FP64)
-// uh: every particle has the same h
+// uh: every particle has the same h; uc: also the same sound speed cs_uni
 void launch_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n, int solid,
                        double dt, bool fuse, float cs32, bool uh);
 void launch_rates_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         int quirks, float cs32, bool uh);
 void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        double alpha, double beta, float cs32, bool uh, const StatsFold& fold = {});
+                        double alpha, double beta, float cs32, bool uh, bool uc, double cs_uni,
+                        const StatsFold& fold = {});
 void launch_cond_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
                        double h_conv, double dt, bool leap, bool first, float cs32, bool uh);
 // conduction of this step fused with the density pass (+ update) of the

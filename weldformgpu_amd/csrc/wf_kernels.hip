@@ -51,6 +51,20 @@ __device__ __forceinline__ T9 tmul(const T9& a, const T9& b, bool quirk) {
   return r;
 }
 
+// particle i's FP64 acceleration record from s = sigma/rho^2, in the layout
+// in force (the general one's {v, m} is written by the caller)
+__device__ __forceinline__ void accel_record64(const Fields& f, int i, double s0, double s1,
+                                               double s2, double s3, double s4, double s5,
+                                               double rho, double cs) {
+  if (f.arec64u) {
+    f.arec64u[i] = make_double4(s0, s1, rho, 0.0);
+    f.arec64[i] = make_double4(s2, s3, s4, s5);
+  } else {
+    f.arec64[rec_at(f, i, 1)] = make_double4(s0, s1, s2, s3);
+    f.arec64[rec_at(f, i, 2)] = make_double4(s4, s5, rho, cs);
+  }
+}
+
 // Safeguarded Newton for the Johnson-Cook radial return,
 // r(g) = s_trial - 3G g - (A + B (ep+g)^n) rt = 0 on [0, hi], from g0, with
 // rt = rate factor x thermal factor and hi = (s_trial - s_y(ep)) / (3G).
@@ -142,7 +156,7 @@ __global__ __launch_bounds__(kBlock) void k_stress(Fields f, StepParams p, Block
     T9 WT = {W.xx, W.yx, W.zx, W.xy, W.yy, W.zy, W.xz, W.yz, W.zz};
     T9 SRT = tmul(S, WT, qp);
     T9 RS = tmul(W, S, qp);
-    if (REC == kRec64)
+    if (REC == kRec64 && !f.arec64u)
       f.arec64[rec_at(f, i, 0)] = make_double4(f.v[0][i], f.v[1][i], f.v[2][i], f.m[i]);
     G = f.G[i];
     const double tr3 = 1.0 / 3.0 * (D.xx + D.yy + D.zz);
@@ -284,9 +298,8 @@ __global__ __launch_bounds__(kBlock) void k_stress(Fields f, StepParams p, Block
     }
     if (REC == kRec64) {  // the same in FP64 for the FP64 acceleration loop
       const double rho = rho_i, ir2 = 1.0 / (rho * rho);
-      f.arec64[rec_at(f, i, 1)] =
-          make_double4(sg[0] * ir2, sg[1] * ir2, sg[2] * ir2, sg[3] * ir2);
-      f.arec64[rec_at(f, i, 2)] = make_double4(sg[4] * ir2, sg[5] * ir2, rho, cs_i);
+      accel_record64(f, i, sg[0] * ir2, sg[1] * ir2, sg[2] * ir2, sg[3] * ir2, sg[4] * ir2,
+                     sg[5] * ir2, rho, cs_i);
     }
     if (ENERGY) {
       double de = f.m[i] / rho_i *
@@ -405,10 +418,10 @@ __global__ __launch_bounds__(kBlock) void k_records64(Fields f, int n) {
   const double4 kv = make_double4(f.v[0][i], f.v[1][i], f.v[2][i], mdj);
   f.kv[i] = kv;
   f.kv_alt[i] = kv;
-  f.arec64[rec_at(f, i, 0)] = make_double4(f.v[0][i], f.v[1][i], f.v[2][i], f.m[i]);
-  f.arec64[rec_at(f, i, 1)] = make_double4(f.sigma[0][i] * ir2, f.sigma[1][i] * ir2,
-                                           f.sigma[2][i] * ir2, f.sigma[3][i] * ir2);
-  f.arec64[rec_at(f, i, 2)] = make_double4(f.sigma[4][i] * ir2, f.sigma[5][i] * ir2, rho, f.Cs[i]);
+  if (!f.arec64u)
+    f.arec64[rec_at(f, i, 0)] = make_double4(f.v[0][i], f.v[1][i], f.v[2][i], f.m[i]);
+  accel_record64(f, i, f.sigma[0][i] * ir2, f.sigma[1][i] * ir2, f.sigma[2][i] * ir2,
+                 f.sigma[3][i] * ir2, f.sigma[4][i] * ir2, f.sigma[5][i] * ir2, rho, f.Cs[i]);
   const double4 tk = make_double4(f.T[i], f.k[i], mdj, 0.0);
   f.tk64[i] = tk;
   f.tk64_alt[i] = tk;

@@ -239,6 +239,23 @@ constexpr int kStage64 = WF_STAGE64;
     z = f.x[2][j];                                                                   \
   }
 
+// LDS layout of a policy whose neighbours are staged whole (k_pair_lds): nv
+// 16-byte and nw (0 or 1) 8- or 4-byte entries a neighbour, each entry its
+// own array of SET.  On a cubic lattice with h = 1.2 dx a tile's staged set
+// holds ~730 particles (at most ~930); under a list skin that reaches the
+// next lattice shell ~760 (at most ~990, 1 % of the tiles above 960).  1,024
+// leave the workgroups a CU that 960 leave, but for the loops with 56 bytes
+// (FP64 density and rates: two instead of three) and 32 (FP32 density, rates
+// and conduction: four instead of five; rates 0.061 against 0.057 ms).
+#define WF_LDS64(nv, nw) \
+  typedef double2 LV;    \
+  typedef double LW;     \
+  static constexpr int NV = nv, NW = nw, SET = 16 * nv + 8 * nw == 56 ? 960 : 1024;
+#define WF_LDS32(nv, nw) \
+  typedef float4 LV;     \
+  typedef float LW;      \
+  static constexpr int NV = nv, NW = nw, SET = 16 * nv + 4 * nw == 32 ? 960 : 1024;
+
 // ---------------------------------------------------------------------------
 // FP64 pair loops (WF_FP64) on the gather kernel below: FP64 positions of the
 // staged set in LDS, the neighbour fields from packed FP64 records.  Each
@@ -260,7 +277,7 @@ struct DensD {
     int mdj_alt;  // write m/rho into the next conduction record (fused with conduction)
   };
   struct Own {
-    double x, y, z, vx, vy, vz, rho;
+    double x, y, z, vx, vy, vz, rho, m;
     HConst hc;
   };
   struct Nb {
@@ -280,6 +297,7 @@ struct DensD {
     o.x = f.x[0][i]; o.y = f.x[1][i]; o.z = f.x[2][i];
     o.vx = f.v[0][i]; o.vy = f.v[1][i]; o.vz = f.v[2][i];
     o.rho = f.rho[i];
+    o.m = f.m[i];  // of the update after the loop
     o.hc = hconst(f.h[i]);
   }
   __device__ static void load(const Fields& f, int j, Nb& nb) {
@@ -295,6 +313,23 @@ struct DensD {
     nb.h = UH ? 0.0 : gat<double>(f.h, j);
   }
 #endif
+  // staged whole: {x, y}, {z, m/rho}, {v_x, v_y}, v_z
+  WF_LDS64(3, 1)
+  __device__ static void lds_put(const Fields& f, int j, const Ctx&, double2 (&q)[3],
+                                 double (&r)[1]) {
+    const double4 v = gat<double4>(f.kv, j);
+    q[0] = make_double2(f.x[0][j], f.x[1][j]);
+    q[1] = make_double2(f.x[2][j], v.w);
+    q[2] = make_double2(v.x, v.y);
+    r[0] = v.z;
+  }
+  __device__ static void lds_get(const double2 (&q)[3], const double (&r)[1], double& x, double& y,
+                                 double& z, Nb& nb) {
+    x = q[0].x;
+    y = q[0].y;
+    z = q[1].x;
+    nb.v = make_double4(q[2].x, q[2].y, r[0], q[1].y);
+  }
   __device__ static void pair(double x, double y, double z, const Nb& nb, const Own& o, Acc& a,
                               const Prm&) {
     const double xx = o.x - x, xy = o.y - y, xz = o.z - z;
@@ -312,7 +347,7 @@ struct DensD {
       if (p.fuse) {
         const double rn = o.rho + p.dt * drho;
         f.rho_alt[i] = rn;
-        const double mdj = f.m[i] / rn;
+        const double mdj = o.m / rn;
         f.kv_alt[i] = make_double4(o.vx, o.vy, o.vz, mdj);
         (p.mdj_alt ? f.tk64_alt : f.tk64)[i].z = mdj;  // m/rho for the conduction loop
       }
@@ -340,6 +375,15 @@ struct RatesD {
   };
   typedef typename DensD<UH>::Nb Nb;
   __device__ static void drop(Nb& nb) { DensD<UH>::drop(nb); }
+  WF_LDS64(3, 1)
+  __device__ static void lds_put(const Fields& f, int j, const Ctx& c, double2 (&q)[3],
+                                 double (&r)[1]) {
+    DensD<UH>::lds_put(f, j, c, q, r);
+  }
+  __device__ static void lds_get(const double2 (&q)[3], const double (&r)[1], double& x, double& y,
+                                 double& z, Nb& nb) {
+    DensD<UH>::lds_get(q, r, x, y, z, nb);
+  }
   struct Acc {
     double dxx, dyy, dzz, dxy, dyz, dxz, wxy, wyz, wxz;
   };
@@ -393,8 +437,9 @@ struct RatesD {
 #ifndef WF_ACCEL64_NBATCH
 #define WF_ACCEL64_NBATCH 2
 #endif
-// BV: the beta (quadratic) viscosity term is on
-template <bool UH, bool BV = false>
+// BV: the beta (quadratic) viscosity term is on; UC: every particle has the
+// same mass and sound speed (and h), so a pair reads neither
+template <bool UH, bool BV = false, bool UC = false>
 struct AccelD {
   WF_GATHER64
   static constexpr int NBATCH = WF_ACCEL64_NBATCH;
@@ -402,6 +447,7 @@ struct AccelD {
     int limit;
     double alpha, beta;
     StatsFold fold;  // the stress pass's statistics, folded by workgroup 0
+    double m_uni, cs_uni;  // UC
   };
   struct Own {
     double x, y, z, vx, vy, vz, di, Ci, s0, s1, s2, s3, s4, s5;
@@ -448,6 +494,36 @@ struct AccelD {
     nb.h = UH ? 0.0 : gat<double>(f.h, j);
   }
 #endif
+  // UC: in LDS {x, y}, {z, rho}, {v_x, v_y}, {v_z, s_xx}, s_yy with s =
+  // sigma/rho^2; gathered {s_zz, s_xy, s_yz, s_xz}
+  WF_LDS64(4, 1)
+  typedef double4 Rest;
+  __device__ static const void* rest(const Fields& f) { return f.arec64; }
+  __device__ static void lds_put(const Fields& f, int j, const Ctx&, double2 (&q)[4],
+                                 double (&r)[1]) {
+    const double4 v = gat<double4>(f.kv, j), s = gat<double4>(f.arec64u, j);
+    q[0] = make_double2(f.x[0][j], f.x[1][j]);
+    q[1] = make_double2(f.x[2][j], s.z);
+    q[2] = make_double2(v.x, v.y);
+    q[3] = make_double2(v.z, s.x);
+    r[0] = s.y;
+  }
+  __device__ static void lds_get(const double2 (&q)[4], const double (&r)[1], double& x, double& y,
+                                 double& z, Nb& nb) {
+    x = q[0].x;
+    y = q[0].y;
+    z = q[1].x;
+    nb.v = make_double4(q[2].x, q[2].y, q[3].x, 0.0);
+    nb.sa.x = q[3].y;
+    nb.sa.y = r[0];
+    nb.sb.z = q[1].y;
+  }
+  __device__ static void rest_get(const Rest& s, Nb& nb) {
+    nb.sa.z = s.x;
+    nb.sa.w = s.y;
+    nb.sb.x = s.z;
+    nb.sb.y = s.w;
+  }
   __device__ static void pair(double x, double y, double z, const Nb& nb, const Own& o, Acc& a,
                               const Prm& p) {
     const double xx = o.x - x, xy = o.y - y, xz = o.z - z;
@@ -463,21 +539,30 @@ struct AccelD {
     const double vn = fmin(vdx, 0.0);
     const double rs = o.di + nb.sb.z;
     const double inv = rcp_f64((r2 + 0.01 * h_ * h_) * rs);
+    const double Cj = UC ? p.cs_uni : nb.sb.w;
     double PI;
     if constexpr (BV) {
-      const double coef = (0.5 * p.alpha) * (o.Ci + nb.sb.w) + p.beta * (h_ * vn * rs * inv);
+      const double coef = (0.5 * p.alpha) * (o.Ci + Cj) + p.beta * (h_ * vn * rs * inv);
       PI = 2.0 * h_ * vn * coef * inv;
     } else {
-      PI = vn * ((h_ * p.alpha) * (o.Ci + nb.sb.w)) * inv;
+      PI = vn * ((h_ * p.alpha) * (o.Ci + Cj)) * inv;
     }
-    const double g = GK * nb.v.w;
+    const double g = GK * (UC ? p.m_uni : nb.v.w);
     const double gx = g * xx, gy = g * xy, gz = g * xz;
     const double mxx = o.s0 + nb.sa.x + PI, myy = o.s1 + nb.sa.y + PI;
     const double mzz = o.s2 + nb.sa.z + PI;
     const double mxy = o.s3 + nb.sa.w, myz = o.s4 + nb.sb.x, mxz = o.s5 + nb.sb.y;
-    a.ax += mxx * gx + mxy * gy + mxz * gz;
-    a.ay += mxy * gx + myy * gy + myz * gz;
-    a.az += mxz * gx + myz * gy + mzz * gz;
+    if constexpr (UC && !BV) {
+      // the order of the general loop's contraction, so that a record layout
+      // does not change the sums
+      a.ax += __builtin_fma(mxz, gz, __builtin_fma(mxy, gy, mxx * gx));
+      a.ay += __builtin_fma(myz, gz, __builtin_fma(mxy, gx, myy * gy));
+      a.az += __builtin_fma(mzz, gz, __builtin_fma(myz, gy, mxz * gx));
+    } else {
+      a.ax += mxx * gx + mxy * gy + mxz * gz;
+      a.ay += mxy * gx + myy * gy + myz * gz;
+      a.az += mxz * gx + myz * gy + mzz * gz;
+    }
   }
   __device__ static void finish(const Fields& f, int i, bool act, const Own&, const Acc& a,
                                 const Prm&) {
@@ -487,6 +572,37 @@ struct AccelD {
     f.a[2][i] = a.az;
   }
 };
+
+// What a conduction pass reads of its own particle after the pair loop, read
+// before it so that the loads are in flight while the pairs are summed
+struct CondIn {
+  double rho, cp, qp, qf, ta;
+  int bct;
+  __device__ __forceinline__ void load(const Fields& f, int i) {
+    rho = f.rho[i];
+    cp = f.cp[i];
+    qp = f.qpl[i];
+    qf = f.qfric[i];
+    ta = f.Ta[i];
+    bct = f.BC_T[i];
+  }
+};
+// dT_i/dt from the conduction sum q: convection (Thermal.cu:36-64), plastic
+// and friction heat, fixed temperature
+template <class P>
+__device__ __forceinline__ double cond_rate(const Fields& f, int i, double q, double Ti,
+                                            const P& p, const CondIn& in) {
+  double acc = q * (1. / (in.rho * in.cp));
+  if (in.bct == WF_BCT_CONVECTION) {
+    const double mi = f.m[i];
+    const double dS2 = pow(mi / in.rho, 0.666666666);
+    const double q_conv = p.h_conv * dS2 * (p.T_inf - Ti) / mi;
+    acc += 1. / in.cp * q_conv;
+  }
+  if (in.qp != 0.0) acc += in.qp * (1. / (in.rho * in.cp));
+  if (in.qf != 0.0) acc += in.qf / (f.m[i] * in.cp);
+  return in.bct == WF_BCT_FIXED ? 0.0 : acc;
+}
 
 // G: conduction dT_i/dt = 1/(rho_i cp_i) sum_j (m_j/rho_j) 4 k_i k_j/(k_i+k_j)
 // (T_i - T_j) GK  (Thermal.cu:101-142, where x_ij.(GK x_ij)/r^2 = GK), then
@@ -504,6 +620,7 @@ struct CondD {
   struct Own {
     double x, y, z, k, T, mdj;
     HConst hc;
+    CondIn in;
   };
   struct Nb {
     double4 tk;  // T, k, m/rho
@@ -523,6 +640,7 @@ struct CondD {
     o.k = f.k[i]; o.T = f.T[i];
     o.mdj = f.tk64[i].z;
     o.hc = hconst(f.h[i]);
+    o.in.load(f, i);
   }
   __device__ static void load(const Fields& f, int j, Nb& nb) {
     nb.tk = gat<double4>(f.tk64, j);
@@ -537,6 +655,22 @@ struct CondD {
     nb.h = UH ? 0.0 : gat<double>(f.h, j);
   }
 #endif
+  // staged whole: {x, y}, {z, m/rho}, {T, k}
+  WF_LDS64(3, 0)
+  __device__ static void lds_put(const Fields& f, int j, const Ctx&, double2 (&q)[3],
+                                 double (&)[1]) {
+    const double4 tk = gat<double4>(f.tk64, j);
+    q[0] = make_double2(f.x[0][j], f.x[1][j]);
+    q[1] = make_double2(f.x[2][j], tk.z);
+    q[2] = make_double2(tk.x, tk.y);
+  }
+  __device__ static void lds_get(const double2 (&q)[3], const double (&)[1], double& x, double& y,
+                                 double& z, Nb& nb) {
+    x = q[0].x;
+    y = q[0].y;
+    z = q[1].x;
+    nb.tk = make_double4(q[2].x, q[2].y, q[1].y, 0.0);
+  }
   __device__ static void pair(double x, double y, double z, const Nb& nb, const Own& o, Acc& a,
                               const Prm&) {
     const double xx = o.x - x, xy = o.y - y, xz = o.z - z;
@@ -544,26 +678,14 @@ struct CondD {
     double rinv, h_;
     const double GK = gk_pair(r2, UH ? o.hc.h : nb.h, o.hc, rinv, h_);
     const double kj = nb.tk.y;
-    const double kh = (kj == o.k) ? 2.0 * o.k : 4.0 * o.k * kj / (o.k + kj);
+    double kh = 2.0 * o.k;  // equal conductivities need no division
+    if (__builtin_expect(kj != o.k, 0)) kh = 4.0 * o.k * kj / (o.k + kj);
     a.q += nb.tk.z * kh * (o.T - nb.tk.x) * GK;
   }
   __device__ static void finish(const Fields& f, int i, bool act, const Own& o, const Acc& a,
                                 const Prm& p) {
     if (!act) return;
-    const double rhoi = f.rho[i], cpi = f.cp[i];
-    double acc = a.q * (1. / (rhoi * cpi));
-    const int bct = f.BC_T[i];
-    if (bct == WF_BCT_CONVECTION) {
-      double mi = f.m[i];
-      double dS2 = pow(mi / rhoi, 0.666666666);
-      double q_conv = p.h_conv * dS2 * (p.T_inf - o.T) / mi;
-      acc += 1. / cpi * q_conv;
-    }
-    double qp = f.qpl[i];
-    if (qp != 0.0) acc += qp * (1. / (rhoi * cpi));
-    const double qf = f.qfric[i];
-    if (qf != 0.0) acc += qf / (f.m[i] * cpi);
-    if (bct == WF_BCT_FIXED) acc = 0.0;
+    const double acc = cond_rate(f, i, a.q, o.T, p, o.in);
     f.dTdt[i] = acc;
     if (p.leap) {
       double Tn;
@@ -571,7 +693,7 @@ struct CondD {
         f.Ta[i] = o.T - p.dt / 2.0 * acc;
         Tn = o.T;
       } else {
-        double ta = f.Ta[i];
+        const double ta = o.in.ta;
         f.Tb[i] = ta;
         double tan = ta + acc * p.dt;
         f.Ta[i] = tan;
@@ -1016,6 +1138,227 @@ void k_pair_gather(Fields f, TileLists tl, typename K::Prm prm) {
   }
 }
 
+
+// ---------------------------------------------------------------------------
+// The pair loops with the neighbours staged whole: everything a pair reads of
+// its neighbour is in LDS, each 16-byte (and one 8- or 4-byte) entry in an
+// array of its own, so a pair costs LDS reads only.  A gather of a record per
+// pair costs the CU's address unit 30-40 cycles per 64 lanes and 16 bytes
+// where an LDS read costs 8-20, and every particle of a tile's set is read
+// once instead of once per pair that has it (about ten times).  The set is
+// LDS-limited (ST entries): two workgroups a CU in the FP64 conduction +
+// density and acceleration loops, three in the others, which measured more
+// than the four and more of the gathering kernel.  Measured on a 759k-particle
+// cylinder (ms, gathering -> staged whole): FP64 conduction + density 0.227
+// -> 0.142, rates 0.123 -> 0.115, acceleration 0.266 -> 0.223, density 0.121
+// -> 0.104; mixed acceleration + integration 0.158 -> 0.136, conduction +
+// density 0.106 -> 0.093, rates 0.061 -> 0.057.  Tiles of 64 particles (four
+// workgroups a CU, but a third more staging) were slower: FP64 step 0.66 ms
+// against 0.59.
+//
+// A policy whose entry would not leave two workgroups a CU keeps the rest of
+// it in a record of its own (typedef Rest, rest(f) the array, rest_get(rest,
+// nb)), which the lane pairs gather together (coload_rec): the FP64
+// acceleration stages 72 of its 104 bytes.  All of it in LDS (one workgroup a
+// CU) took 0.264 ms.
+//
+// The lanes and their sums are those of k_pair_gather; P of the tile's
+// kTileP particles make a workgroup.
+template <class K, class = void>
+struct HasLds {
+  static constexpr bool on = false;
+};
+template <class K>
+struct HasLds<K, std::void_t<typename K::LV>> {
+  static constexpr bool on = true;
+};
+template <class K, class = void>
+struct RestOf {
+  static constexpr bool on = false;
+  typedef int type;
+};
+template <class K>
+struct RestOf<K, std::void_t<typename K::Rest>> {
+  static constexpr bool on = true;
+  typedef typename K::Rest type;
+};
+template <class K, int L, int P>
+__global__ __launch_bounds__(L * P) void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
+  constexpr int S = kTileP / P, NT = L * P, ST = K::SET;
+  static_assert(L >= 2 && L <= 16 && (L & (L - 1)) == 0, "a power of two of lanes per particle");
+  typedef typename K::LV LV;
+  typedef typename K::LW LW;
+  typedef typename K::PT PT;
+  constexpr int NV = K::NV, NW = K::NW;
+  constexpr bool R = RestOf<K>::on;
+  typedef typename RestOf<K>::type Rest;
+  __shared__ LV sv[NV][ST];
+  __shared__ LW sw[NW > 0 ? ST : 1];
+  __shared__ int sj[R ? ST : 1];
+  const int b = xcd_tile(blockIdx.x, gridDim.x);
+  const int t = b / S;
+  const int tid = threadIdx.x;
+  const int sub = tid & (L - 1);
+  const int i = b * P + tid / L;
+  const bool act = i < prm.limit;
+  const int ub = tl.uoff[t], ucnt = tl.ucnt[t];
+  const int* __restrict__ tj = tl.tj + ub;
+  const int cnt = act ? tl.count[i] : 0;
+  const typename K::Ctx cx = K::ctx(f, t, prm);
+  typename K::Own own;
+  typename K::Acc acc;
+  K::init(f, i, act, own, acc, cx);
+  // SU neighbours per thread at a time: their indices, then everything the
+  // pairs read of them, then the LDS writes
+  auto stage = [&](int c0, int m) {
+    constexpr int SU = 4;
+    for (int s0 = tid; s0 < m; s0 += SU * NT) {
+      int jj[SU];
+#pragma unroll
+      for (int u = 0; u < SU; u++) jj[u] = s0 + u * NT < m ? tj[c0 + s0 + u * NT] : 0;
+      LV q[SU][NV];
+      LW r[SU][1];
+#pragma unroll
+      for (int u = 0; u < SU; u++) K::lds_put(f, jj[u], cx, q[u], r[u]);
+#pragma unroll
+      for (int u = 0; u < SU; u++) {
+        const int s = s0 + u * NT;
+        if (s < m) {
+#pragma unroll
+          for (int v = 0; v < NV; v++) sv[v][s] = q[u][v];
+          if constexpr (NW > 0) sw[s] = r[u][0];
+          if constexpr (R) sj[s] = jj[u];
+        }
+      }
+    }
+  };
+  auto fetch = [&](int sl, PT& x, PT& y, PT& z, typename K::Nb& nb) {
+    LV q[NV];
+    LW r[1] = {};
+#pragma unroll
+    for (int v = 0; v < NV; v++) q[v] = sv[v][sl];
+    if constexpr (NW > 0) r[0] = sw[sl];
+    K::lds_get(q, r, x, y, z, nb);
+  };
+  // body(sum) adds the pairs of a quad, through the policy's partial sums if
+  // it has them
+  auto quad = [&](auto&& body) {
+    if constexpr (PartOf<K>::on) {
+      typename K::Part part;
+      K::pzero(part);
+      body(part);
+      K::flush(acc, part);
+    } else {
+      body(acc);
+    }
+  };
+  if (ucnt <= ST) {
+    stage(0, ucnt);
+    __syncthreads();
+    // lanes past the padded particle range read row 0 of the last particle
+    // (their lists are empty); rows are clamped into the list
+    const uint2* __restrict__ q = tl.slotq + min((int64_t)i, tl.npad - 1);
+    const int klast = max(cnt - 1, 0);
+    // 32-bit word index: rows x npad stays below 2^32 (kMaxParticles)
+    const unsigned np = (unsigned)tl.npad;
+    auto word = [&](int k) { return q[(unsigned)(min(k, klast) >> 2) * np]; };
+    auto sl_of = [](const uint2 w, int u) {
+      const unsigned h = (u & 2) ? w.y : w.x;
+      return (int)((u & 1) ? h >> 16 : h & 0xFFFFu);
+    };
+    constexpr int KS = 4 * L;  // slots from one of the lane's quads to its next
+    const int k0 = 4 * sub;
+    // with a gathered rest both lanes of a pair run the same steps (coload_rec)
+    const int kend = R ? (cnt + KS - 1) / KS * KS + k0 : cnt;
+    uint2 w0 = word(k0), w1 = word(k0 + KS);
+    int jn[4];
+    if constexpr (R) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) jn[u] = k0 + u < cnt ? sj[sl_of(w0, u)] : 0;
+    }
+    for (int k = k0; k < kend; k += KS) {
+      const int nk = min(4, cnt - k);
+      int jc[4];
+      if constexpr (R) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) jc[u] = jn[u];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (k + KS + u < cnt) jn[u] = sj[sl_of(w1, u)];
+      }
+      const uint2 w2 = word(k + 2 * KS);
+      Rest rr[4];
+      if constexpr (R) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          uint4 c[sizeof(Rest) / 16];
+          coload_rec<sizeof(Rest) / 16>(K::rest(f), jc[u], sub & 1, c);
+          __builtin_memcpy(&rr[u], c, sizeof(Rest));
+        }
+      }
+      quad([&](auto& sum) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          PT x, y, z;
+          typename K::Nb nb;
+          if constexpr (DropOf<K>::on) {
+            // entries past the list add exact zeros (drop)
+            fetch(u < nk ? sl_of(w0, u) : 0, x, y, z, nb);
+            if (u >= nk) K::drop(nb);
+            K::pair(x, y, z, nb, own, sum, prm);
+          } else if (u < nk) {
+            fetch(sl_of(w0, u), x, y, z, nb);
+            if constexpr (R) K::rest_get(rr[u], nb);
+            K::pair(x, y, z, nb, own, sum, prm);
+          }
+        }
+      });
+      w0 = w1;
+      w1 = w2;
+    }
+  } else {
+    // a larger set in passes; each lane takes the list entries of its quads
+    // that fall in the pass
+    SlotReader sr;
+    sr.init(tl, i, cnt);
+    for (int c0 = 0; c0 < ucnt; c0 += ST) {
+      const int m = min(ST, ucnt - c0);
+      __syncthreads();
+      stage(c0, m);
+      __syncthreads();
+      const int lim = c0 + m;
+      while (sr.k < sr.cnt) {
+        if (((sr.k >> 2) & (L - 1)) != sub) {
+          sr.skip_quad();
+          continue;
+        }
+        const int sl = sr.slot();
+        if (sl >= lim) break;
+        sr.advance();
+        quad([&](auto& sum) {
+          PT x, y, z;
+          typename K::Nb nb;
+          fetch(sl - c0, x, y, z, nb);
+          if constexpr (R) K::rest_get(gat<Rest>(K::rest(f), sj[sl - c0]), nb);
+          K::pair(x, y, z, nb, own, sum, prm);
+        });
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 1; m < L; m <<= 1) {
+    const typename K::Acc other = lane_value_xor(acc, m);
+    K::merge(acc, other);
+  }
+  if (sub == 0) K::finish(f, i, act, own, acc, prm);
+  if constexpr (FoldOf<K>::on) {
+    if (blockIdx.x == 0 && prm.fold.nb > 0) {
+      __syncthreads();  // the staged set is read no more: its LDS is scratch
+      block_fold_stats(prm.fold, reinterpret_cast<unsigned long long*>(&sv[0][0]));
+    }
+  }
+}
+
 // A: density rate (InteractionAlt.cu:166-246), fused density update writes
 // the next {v, m/rho} mirror
 template <bool UH>
@@ -1032,6 +1375,7 @@ struct DensG {
   struct Own {
     float x, y, z, vx, vy, vz;
     HConstF hc;
+    double rho, m;  // of the update after the loop
   };
   struct Nb {
     float4 v;  // v, m/rho
@@ -1052,10 +1396,28 @@ struct DensG {
     const float4 v = f.v4[i];
     o.vx = v.x; o.vy = v.y; o.vz = v.z;
     o.hc = hconst_f(f.h32[i]);
+    o.rho = f.rho[i];
+    o.m = f.m[i];
   }
   __device__ static void load(const Fields& f, int j, Nb& nb) {
     nb.v = gat<float4>(f.v4, j);
     nb.h = UH ? 0.f : gat<float>(f.h32, j);
+  }
+  // staged whole: {x, y, z, m/rho}, {v, -}
+  WF_LDS32(2, 0)
+  __device__ static void lds_put(const Fields& f, int j, const Ctx& c, float4 (&q)[2],
+                                 float (&)[1]) {
+    float x, y, z;
+    pos32(f, j, c, x, y, z);
+    q[1] = gat<float4>(f.v4, j);
+    q[0] = make_float4(x, y, z, q[1].w);
+  }
+  __device__ static void lds_get(const float4 (&q)[2], const float (&)[1], float& x, float& y,
+                                 float& z, Nb& nb) {
+    x = q[0].x;
+    y = q[0].y;
+    z = q[0].z;
+    nb.v = make_float4(q[1].x, q[1].y, q[1].z, q[0].w);
   }
   __device__ static void pair(float x, float y, float z, const Nb& nb, const Own& o, Part& a,
                               const Prm&) {
@@ -1066,19 +1428,18 @@ struct DensG {
     const float vx = o.vx - nb.v.x, vy = o.vy - nb.v.y, vz = o.vz - nb.v.z;
     a = __builtin_fmaf(nb.v.w, GK * (vx * xx + vy * xy + vz * xz), a);
   }
-  __device__ static void finish(const Fields& f, int i, bool act, const Own&, const Acc& a,
+  __device__ static void finish(const Fields& f, int i, bool act, const Own& o, const Acc& a,
                                 const Prm& p) {
     if (act) {
-      const double rho = f.rho[i];
+      const double rho = o.rho;
       const double drho = rho * a.val();
       f.drho[i] = drho;
       if (p.fuse) {
         const double rn = rho + p.dt * drho;
         f.rho_alt[i] = rn;
-        float4 v = f.v4[i];
-        v.w = (float)(f.m[i] / rn);
-        f.v4_alt[i] = v;
-        (p.mdj_alt ? f.tk4_alt : f.tk4)[i].z = v.w;  // m/rho for the conduction loop
+        const float mdj = (float)(o.m / rn);
+        f.v4_alt[i] = make_float4(o.vx, o.vy, o.vz, mdj);
+        (p.mdj_alt ? f.tk4_alt : f.tk4)[i].z = mdj;  // m/rho for the conduction loop
       }
     } else if (p.fuse && i < p.n) {
       f.rho_alt[i] = f.rho[i];
@@ -1116,6 +1477,15 @@ struct RatesG {
   __device__ static void put(Nb& nb, const Extra& e) { nb.v = e; }
   __device__ static void load(const Fields& f, int j, Nb& nb) {
     nb.h = UH ? 0.f : gat<float>(f.h32, j);
+  }
+  WF_LDS32(2, 0)
+  __device__ static void lds_put(const Fields& f, int j, const Ctx& c, float4 (&q)[2],
+                                 float (&r)[1]) {
+    DensG<UH>::lds_put(f, j, c, q, r);
+  }
+  __device__ static void lds_get(const float4 (&q)[2], const float (&r)[1], float& x, float& y,
+                                 float& z, Nb& nb) {
+    DensG<UH>::lds_get(q, r, x, y, z, nb);
   }
   // products a_k x_l: xx, yy, zz, then (x y, y x), (y z, z y), (x z, z x)
   // each product of two FP32 factors is exact in FP64 and added by one FP64
@@ -1185,7 +1555,8 @@ struct RatesG {
 // BV: the beta (quadratic) viscosity term is on; IT: each particle is
 // integrated as soon as its sum is done (IntegratePrm), its integration
 // inputs loaded before the pair loop
-template <bool UH, bool BV = false, bool IT = false>
+// UC: every particle has the same sound speed (and h)
+template <bool UH, bool BV = false, bool IT = false, bool UC = false>
 struct AccelG {
   WF_GATHER32
   static constexpr int NBATCH = WF_ACCEL32_NBATCH;
@@ -1196,6 +1567,7 @@ struct AccelG {
     float cs;
     IntegratePrm ip;  // integrate each particle after its sum (IT)
     StatsFold fold;   // the stress pass's statistics, folded by workgroup 0
+    float cs_uni;     // UC
   };
   struct NoIn {};
   struct Own {
@@ -1243,6 +1615,31 @@ struct AccelG {
     return v;
   }
   __device__ static void put(Nb& nb, const Extra& e) { nb.v = e; }
+  // UC: staged whole: {x, y, z, rho}, {v, s_xx}, {s_yy, s_zz, s_xy, s_yz},
+  // {s_xz, m} with s = sigma/rho^2 (56 bytes: 960 leave three workgroups a CU)
+  typedef float4 LV;
+  typedef float2 LW;
+  static constexpr int NV = 3, NW = 1, SET = 960;
+  __device__ static void lds_put(const Fields& f, int j, const Ctx& c, float4 (&q)[3],
+                                 float2 (&r)[1]) {
+    const float4 v = gat<float4>(f.v4, j);
+    const float4 sa = gat<float4, 32>(f.arec, j), sb = gat<float4, 32>(f.arec, j, 16);
+    float x, y, z;
+    pos32(f, j, c, x, y, z);
+    q[0] = make_float4(x, y, z, sb.z);
+    q[1] = make_float4(v.x, v.y, v.z, sa.x);
+    q[2] = make_float4(sa.y, sa.z, sa.w, sb.x);
+    r[0] = make_float2(sb.y, v.w * sb.z);  // m = (m/rho) rho, as extra() forms it
+  }
+  __device__ static void lds_get(const float4 (&q)[3], const float2 (&r)[1], float& x, float& y,
+                                 float& z, Nb& nb) {
+    x = q[0].x;
+    y = q[0].y;
+    z = q[0].z;
+    nb.v = make_float4(q[1].x, q[1].y, q[1].z, r[0].y);
+    nb.sa = make_float4(q[1].w, q[2].x, q[2].y, q[2].z);
+    nb.sb = make_float4(q[2].w, r[0].x, q[0].w, 0.f);
+  }
   __device__ static void load(const Fields& f, int j, Nb& nb) {
     nb.sa = gat<float4, 32>(f.arec, j);  // rec32_at(j, 0..1)
     nb.sb = gat<float4, 32>(f.arec, j, 16);
@@ -1265,13 +1662,14 @@ struct AccelG {
     const float vn = fminf(vdx, 0.f);
     const float rs = o.di + nb.sb.z;
     const float inv = __builtin_amdgcn_rcpf((r2 + 0.01f * h_ * h_) * rs);
+    const float Cj = UC ? p.cs_uni : nb.sb.w;
     float PI;
     if constexpr (BV) {
       const float coef =
-          (0.5f * p.alpha32) * (o.Ci + nb.sb.w) + p.beta32 * (h_ * vn * rs * inv);
+          (0.5f * p.alpha32) * (o.Ci + Cj) + p.beta32 * (h_ * vn * rs * inv);
       PI = 2.f * h_ * vn * coef * inv;
     } else {
-      PI = vn * ((h_ * p.alpha32) * (o.Ci + nb.sb.w)) * inv;
+      PI = vn * ((h_ * p.alpha32) * (o.Ci + Cj)) * inv;
     }
     const float g = GK * nb.v.w;
     const float gx = g * xx, gy = g * xy, gz = g * xz;
@@ -1311,6 +1709,8 @@ struct CondG {
   struct Own {
     float x, y, z, k, T, mdj;
     HConstF hc;
+    CondIn in;
+    double Ti;
   };
   struct Nb {
     float4 tk;  // T, k, m/rho
@@ -1333,6 +1733,8 @@ struct CondG {
     o.k = tk.y;
     o.mdj = tk.z;
     o.hc = hconst_f(f.h32[i]);
+    o.in.load(f, i);
+    o.Ti = f.T[i];
   }
   // the neighbour's {T, k, m/rho} is staged in LDS with its position (the
   // pass writes only the next record, tk4_alt)
@@ -1341,6 +1743,22 @@ struct CondG {
   __device__ static void put(Nb& nb, const Extra& e) { nb.tk = e; }
   __device__ static void load(const Fields& f, int j, Nb& nb) {
     nb.h = UH ? 0.f : gat<float>(f.h32, j);
+  }
+  // staged whole: {x, y, z, m/rho}, {T, k, -, -}
+  WF_LDS32(2, 0)
+  __device__ static void lds_put(const Fields& f, int j, const Ctx& c, float4 (&q)[2],
+                                 float (&)[1]) {
+    float x, y, z;
+    pos32(f, j, c, x, y, z);
+    q[1] = gat<float4>(f.tk4, j);
+    q[0] = make_float4(x, y, z, q[1].z);
+  }
+  __device__ static void lds_get(const float4 (&q)[2], const float (&)[1], float& x, float& y,
+                                 float& z, Nb& nb) {
+    x = q[0].x;
+    y = q[0].y;
+    z = q[0].z;
+    nb.tk = make_float4(q[1].x, q[1].y, q[0].w, 0.f);
   }
   __device__ static void pair(float x, float y, float z, const Nb& nb, const Own& o, Part& a,
                               const Prm&) {
@@ -1355,20 +1773,7 @@ struct CondG {
   __device__ static void finish(const Fields& f, int i, bool act, const Own& o, const Acc& a,
                                 const Prm& p) {
     if (!act) return;
-    const double rhoi = f.rho[i], cpi = f.cp[i], Ti = f.T[i];
-    double acc = a.val() * (1. / (rhoi * cpi));
-    const int bct = f.BC_T[i];
-    if (bct == WF_BCT_CONVECTION) {
-      double mi = f.m[i];
-      double dS2 = pow(mi / rhoi, 0.666666666);
-      double q_conv = p.h_conv * dS2 * (p.T_inf - Ti) / mi;
-      acc += 1. / cpi * q_conv;
-    }
-    double qp = f.qpl[i];
-    if (qp != 0.0) acc += qp * (1. / (rhoi * cpi));
-    const double qf = f.qfric[i];
-    if (qf != 0.0) acc += qf / (f.m[i] * cpi);
-    if (bct == WF_BCT_FIXED) acc = 0.0;
+    const double Ti = o.Ti, acc = cond_rate(f, i, a.val(), Ti, p, o.in);
     f.dTdt[i] = acc;
     if (p.leap) {
       double Tn;
@@ -1376,7 +1781,7 @@ struct CondG {
         f.Ta[i] = Ti - p.dt / 2.0 * acc;
         Tn = Ti;
       } else {
-        double ta = f.Ta[i];
+        const double ta = o.in.ta;
         f.Tb[i] = ta;
         double tan = ta + acc * p.dt;
         f.Ta[i] = tan;
@@ -1531,37 +1936,6 @@ struct SurfG {
   }
 };
 
-void launch_surface_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                          double ntot, double totmass, int id_free_surf, double r2cut, bool um,
-                          double m_value, float cs32) {
-  if (solid <= 0) return;
-  const float r2 = (float)r2cut;
-  if (um) {
-    const SurfG<true>::Prm p{solid, id_free_surf, ntot, totmass, r2, (float)m_value, cs32};
-    hipLaunchKernelGGL(k_pair_gather<SurfG<true>>, dim3(ntiles(solid)),
-                       dim3(kTileP * SurfG<true>::LANES), 0, s, f, tl, p);
-  } else {
-    const SurfG<false>::Prm p{solid, id_free_surf, ntot, totmass, r2, 0.f, cs32};
-    hipLaunchKernelGGL(k_pair_gather<SurfG<false>>, dim3(ntiles(solid)),
-                       dim3(kTileP * SurfG<false>::LANES), 0, s, f, tl, p);
-  }
-}
-
-void launch_surface_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                          double ntot, double totmass, int id_free_surf, double r2cut, bool um,
-                          double m_value) {
-  if (solid <= 0) return;
-  if (um) {
-    const SurfD<true>::Prm p{solid, id_free_surf, ntot, totmass, r2cut, m_value};
-    hipLaunchKernelGGL(k_pair_gather<SurfD<true>>, dim3(ntiles(solid)), dim3(kTileP * SurfD<true>::LANES), 0, s, f,
-                       tl, p);
-  } else {
-    const SurfD<false>::Prm p{solid, id_free_surf, ntot, totmass, r2cut, 0.0};
-    hipLaunchKernelGGL(k_pair_gather<SurfD<false>>, dim3(ntiles(solid)), dim3(kTileP * SurfD<false>::LANES), 0, s, f,
-                       tl, p);
-  }
-}
-
 }  // namespace wf
 
 namespace wf {
@@ -1666,6 +2040,44 @@ struct CondDens : FusedExtra<A, CondDensNb<A, B>>, FusedPart<A, B>, FusedDrop<A,
       B::coload(f, j, sub, nb.b);
     }
   }
+  // staged whole: the density pass's entries and T, k (the m/rho of the two
+  // records is the same value): FP64 {x, y}, {z, m/rho}, {v_x, v_y}, {T, k},
+  // v_z, FP32 {x, y, z, m/rho}, {v, T}, k
+  static constexpr bool F64 = std::is_same<PT, double>::value;
+  typedef std::conditional_t<F64, double2, float4> LV;
+  typedef PT LW;
+  static constexpr int NV = F64 ? 4 : 2, NW = 1, SET = 1024;
+  __device__ static void lds_put(const Fields& f, int j, const Ctx& c, LV (&q)[NV], PT (&r)[1]) {
+    if constexpr (F64) {
+      const double4 v = gat<double4>(f.kv, j);
+      q[0] = make_double2(f.x[0][j], f.x[1][j]);
+      q[1] = make_double2(f.x[2][j], v.w);
+      q[2] = make_double2(v.x, v.y);
+      q[3] = gat<double2, 32>(f.tk64, j);
+      r[0] = v.z;
+    } else {
+      const float4 v = gat<float4>(f.v4, j), tk = gat<float4>(f.tk4, j);
+      float x, y, z;
+      pos32(f, j, c, x, y, z);
+      q[0] = make_float4(x, y, z, v.w);
+      q[1] = make_float4(v.x, v.y, v.z, tk.x);
+      r[0] = tk.y;
+    }
+  }
+  __device__ static void lds_get(const LV (&q)[NV], const PT (&r)[1], PT& x, PT& y, PT& z,
+                                 Nb& nb) {
+    x = q[0].x;
+    y = q[0].y;
+    if constexpr (F64) {
+      z = q[1].x;
+      nb.b.v = make_double4(q[2].x, q[2].y, r[0], q[1].y);
+      nb.a.tk = make_double4(q[3].x, q[3].y, q[1].y, 0.0);
+    } else {
+      z = q[0].z;
+      nb.b.v = make_float4(q[1].x, q[1].y, q[1].z, q[0].w);
+      nb.a.tk = make_float4(q[1].w, r[0], q[0].w, 0.f);
+    }
+  }
   // S: the sums (Acc) or the batch's partial sums (Part)
   template <class S>
   __device__ static void pair(PT x, PT y, PT z, const Nb& nb, const Own& o, S& a,
@@ -1689,26 +2101,29 @@ using CondDensD = CondDens<CondD<UH>, DensD<UH>>;
 template <bool UH>
 using CondDensG = CondDens<CondG<UH>, DensG<UH>>;
 
-// the acceleration loops with the beta viscosity term
-template <bool UH>
-using AccelDB = AccelD<UH, true>;
-template <bool UH>
-using AccelGB = AccelG<UH, true>;
-
 LaunchEvents g_next_launch = {nullptr, nullptr};
 
-// one pair pass: grid tiles of kTileP particles, K::LANES threads each (with
-// its dispatch timestamps in g_next_launch's events when those are set)
 template <class K>
-static void launch_pair(hipStream_t s, int grid, const Fields& f, const TileLists& tl,
-                        const typename K::Prm& p) {
+static void launch_timed(void (*kernel)(Fields, TileLists, typename K::Prm), dim3 grid, dim3 block,
+                         hipStream_t s, const Fields& f, const TileLists& tl,
+                         const typename K::Prm& p) {
   if (g_next_launch.start) {
-    hipExtLaunchKernelGGL(k_pair_gather<K>, dim3(grid), dim3(kTileP * K::LANES), 0, s,
-                          g_next_launch.start, g_next_launch.stop, 0, f, tl, p);
+    hipExtLaunchKernelGGL(kernel, grid, block, 0, s, g_next_launch.start, g_next_launch.stop, 0, f,
+                          tl, p);
     g_next_launch = LaunchEvents{nullptr, nullptr};
   } else {
-    hipLaunchKernelGGL(k_pair_gather<K>, dim3(grid), dim3(kTileP * K::LANES), 0, s, f, tl, p);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, f, tl, p);
   }
+}
+// one pair pass over nt tiles, the neighbours staged whole (LDS) or gathered
+// (with its dispatch timestamps in g_next_launch's events when those are set)
+template <class K, bool LDS = true>
+static void launch_pair(hipStream_t s, int nt, const Fields& f, const TileLists& tl,
+                        const typename K::Prm& p) {
+  if constexpr (LDS && HasLds<K>::on)
+    launch_timed<K>(k_pair_lds<K, 2, kTileP>, dim3(nt), dim3(2 * kTileP), s, f, tl, p);
+  else
+    launch_timed<K>(k_pair_gather<K>, dim3(nt), dim3(kTileP * K::LANES), s, f, tl, p);
 }
 
 // launch policy POL with every particle's h equal (UH) or not
@@ -1716,7 +2131,34 @@ template <template <bool> class POL, class... A>
 static void launch_gather(hipStream_t s, const Fields& f, const TileLists& tl, int grid, bool uh,
                           A... args) {
   if (uh) launch_pair<POL<true>>(s, grid, f, tl, typename POL<true>::Prm{args...});
-  else launch_pair<POL<false>>(s, grid, f, tl, typename POL<false>::Prm{args...});
+  else launch_pair<POL<false>, false>(s, grid, f, tl, typename POL<false>::Prm{args...});
+}
+
+void launch_surface_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
+                          double ntot, double totmass, int id_free_surf, double r2cut, bool um,
+                          double m_value, float cs32) {
+  if (solid <= 0) return;
+  const float r2 = (float)r2cut;
+  if (um) {
+    const SurfG<true>::Prm p{solid, id_free_surf, ntot, totmass, r2, (float)m_value, cs32};
+    launch_pair<SurfG<true>>(s, ntiles(solid), f, tl, p);
+  } else {
+    const SurfG<false>::Prm p{solid, id_free_surf, ntot, totmass, r2, 0.f, cs32};
+    launch_pair<SurfG<false>, false>(s, ntiles(solid), f, tl, p);
+  }
+}
+
+void launch_surface_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
+                          double ntot, double totmass, int id_free_surf, double r2cut, bool um,
+                          double m_value) {
+  if (solid <= 0) return;
+  if (um) {
+    const SurfD<true>::Prm p{solid, id_free_surf, ntot, totmass, r2cut, m_value};
+    launch_pair<SurfD<true>>(s, ntiles(solid), f, tl, p);
+  } else {
+    const SurfD<false>::Prm p{solid, id_free_surf, ntot, totmass, r2cut, 0.0};
+    launch_pair<SurfD<false>, false>(s, ntiles(solid), f, tl, p);
+  }
 }
 
 void launch_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, int solid,
@@ -1731,27 +2173,50 @@ void launch_rates_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int
   launch_gather<RatesD>(s, f, tl, ntiles(solid), uh, solid, xz);
 }
 void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        double alpha, double beta, bool uh, const StatsFold& fold) {
+                        double alpha, double beta, bool uh, double m_uni, double cs_uni,
+                        const StatsFold& fold) {
   if (solid <= 0) return;
-  if (beta != 0.0) {
-    launch_gather<AccelDB>(s, f, tl, ntiles(solid), uh, solid, alpha, beta, fold);
-  } else {
-    launch_gather<AccelD>(s, f, tl, ntiles(solid), uh, solid, alpha, beta, fold);
-  }
+  auto go = [&](auto tag, auto lds) {
+    typedef decltype(tag) K;
+    const typename K::Prm p{solid, alpha, beta, fold, m_uni, cs_uni};
+    launch_pair<K, lds()>(s, ntiles(solid), f, tl, p);
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  if (f.arec64u)
+    beta != 0.0 ? go(AccelD<true, true, true>{}, yes) : go(AccelD<true, false, true>{}, yes);
+  else if (uh)
+    beta != 0.0 ? go(AccelD<true, true>{}, no) : go(AccelD<true, false>{}, no);
+  else
+    beta != 0.0 ? go(AccelD<false, true>{}, no) : go(AccelD<false, false>{}, no);
+}
+// uc: every particle has the same h and sound speed cs_uni
+template <bool IT>
+static void accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
+                        double alpha, double beta, float cs32, bool uh, bool uc, double cs_uni,
+                        const IntegratePrm& ip, const StatsFold& fold) {
+  if (solid <= 0) return;
+  auto go = [&](auto tag, auto lds) {
+    typedef decltype(tag) K;
+    launch_pair<K, lds()>(s, ntiles(solid), f, tl,
+                          typename K::Prm{solid, (float)alpha, (float)beta, cs32, ip, fold,
+                                          (float)cs_uni});
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  if (uc)
+    beta != 0.0 ? go(AccelG<true, true, IT, true>{}, yes) : go(AccelG<true, false, IT, true>{}, yes);
+  else if (uh)
+    beta != 0.0 ? go(AccelG<true, true, IT>{}, no) : go(AccelG<true, false, IT>{}, no);
+  else
+    beta != 0.0 ? go(AccelG<false, true, IT>{}, no) : go(AccelG<false, false, IT>{}, no);
 }
 void launch_accel_integrate_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                                  double alpha, double beta, float cs32, bool uh, double dt,
-                                  const BcTable& bc, const Frame32& fr, const IntegrateOut& out,
-                                  const StatsFold& fold) {
-  if (solid <= 0) return;
-  const IntegratePrm ip{dt, bc, fr, out};
-  auto go = [&](auto tag) {
-    typedef decltype(tag) K;
-    launch_pair<K>(s, ntiles(solid), f, tl,
-                   typename K::Prm{solid, (float)alpha, (float)beta, cs32, ip, fold});
-  };
-  if (beta != 0.0) uh ? go(AccelG<true, true, true>{}) : go(AccelG<false, true, true>{});
-  else uh ? go(AccelG<true, false, true>{}) : go(AccelG<false, false, true>{});
+                                  double alpha, double beta, float cs32, bool uh, bool uc,
+                                  double cs_uni, double dt, const BcTable& bc, const Frame32& fr,
+                                  const IntegrateOut& out, const StatsFold& fold) {
+  accel_mixed<true>(s, f, tl, solid, alpha, beta, cs32, uh, uc, cs_uni,
+                    IntegratePrm{dt, bc, fr, out}, fold);
 }
 void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
                        double h_conv, double dt, bool leap, bool first, bool uh) {
@@ -1771,14 +2236,9 @@ void launch_rates_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int
   launch_gather<RatesG>(s, f, tl, ntiles(solid), uh, solid, xz, cs32);
 }
 void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        double alpha, double beta, float cs32, bool uh, const StatsFold& fold) {
-  if (solid <= 0) return;
-  if (beta != 0.0)
-    launch_gather<AccelGB>(s, f, tl, ntiles(solid), uh, solid, (float)alpha, (float)beta, cs32,
-                           IntegratePrm{}, fold);
-  else
-    launch_gather<AccelG>(s, f, tl, ntiles(solid), uh, solid, (float)alpha, (float)beta, cs32,
-                          IntegratePrm{}, fold);
+                        double alpha, double beta, float cs32, bool uh, bool uc, double cs_uni,
+                        const StatsFold& fold) {
+  accel_mixed<false>(s, f, tl, solid, alpha, beta, cs32, uh, uc, cs_uni, IntegratePrm{}, fold);
 }
 void launch_cond_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
                        double h_conv, double dt, bool leap, bool first, float cs32, bool uh) {
@@ -1791,27 +2251,27 @@ void launch_cond_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl,
                             bool first, bool uh, const unsigned long long* pz_d2,
                             double pz_skin2) {
   if (n <= 0) return;
-  auto go = [&](auto tag) {
+  auto go = [&](auto tag, auto split) {
     typedef decltype(tag) K;
     const typename K::Prm p{n, {n, T_inf, h_conv, dt, leap ? 1 : 0, first ? 1 : 0},
                             {solid, n, dt, 1, 1}, pz_d2, pz_skin2};
-    launch_pair<K>(s, ntiles(n), f, tl, p);
+    launch_pair<K, split()>(s, ntiles(n), f, tl, p);
   };
-  if (uh) go(CondDensD<true>{});
-  else go(CondDensD<false>{});
+  if (uh) go(CondDensD<true>{}, std::true_type{});
+  else go(CondDensD<false>{}, std::false_type{});
 }
 void launch_cond_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n,
                             int solid, double T_inf, double h_conv, double dt, bool leap,
                             bool first, float cs32, bool uh, const unsigned long long* pz_d2,
                             double pz_skin2) {
   if (n <= 0) return;
-  auto go = [&](auto tag) {
+  auto go = [&](auto tag, auto split) {
     typedef decltype(tag) K;
     const typename K::Prm p{n, {n, T_inf, h_conv, dt, leap ? 1 : 0, first ? 1 : 0, cs32},
                             {solid, n, dt, 1, cs32, 1}, pz_d2, pz_skin2};
-    launch_pair<K>(s, ntiles(n), f, tl, p);
+    launch_pair<K, split()>(s, ntiles(n), f, tl, p);
   };
-  if (uh) go(CondDensG<true>{});
-  else go(CondDensG<false>{});
+  if (uh) go(CondDensG<true>{}, std::true_type{});
+  else go(CondDensG<false>{}, std::false_type{});
 }
 }  // namespace wf
