@@ -4,6 +4,8 @@ They take domains whose particles share one h, and in the acceleration one
 sound speed (FP64: and one mass); other domains keep the gathering loops and
 the general record.  Both must give the same passes at every tile remainder,
 and a domain that changes from one to the other must not use stale records.
+Up to 32, 64 and 128 tiles (4,096, 8,192 and 16,384 particles) a tile is dealt
+out to 8, 4 and 2 workgroups.
 
 Tolerances: against the FP64 oracle, one call, relative L2 <= 1e-12 (FP64:
 rounding of ~56 terms a sum) and 2e-5 (mixed: FP32 terms).
@@ -23,7 +25,7 @@ TOL = {_abi.WF_FP64: 1e-12, _abi.WF_MIXED: 2e-5}
 def _scenario(n, precision, beta):
     """The first n particles of a thermo-mechanical cylinder, random v, stress
     and temperature."""
-    sc = scenarios.c3_johnson_cook(scale=0.2)
+    sc = scenarios.c3_johnson_cook(scale=0.3)
     for k, v in sc.fields.items():
         sc.fields[k] = v[:n].copy()
     sc.cfg.n_particles = sc.cfg.solid_count = n
@@ -50,7 +52,7 @@ def _passes(d, st, cfg, tol):
 
 
 @pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
-@pytest.mark.parametrize("n", [1, 63, 127, 128, 129, 1000, 4481])
+@pytest.mark.parametrize("n", [1, 63, 127, 128, 129, 1000, 4096, 4097, 8192, 8193, 16384, 16385])
 def test_uniform_and_general_passes(oracle, wflib, n, precision):
     sc = _scenario(n, precision, 1.0 if n == 129 else 0.0)
     st = to_oracle(oracle, sc)
@@ -69,4 +71,18 @@ def test_uniform_and_general_passes(oracle, wflib, n, precision):
         for k in ("h", "m", "Cs"):
             st[k] = sc.fields[k]
             d.set(k, sc.fields[k])
+        _passes(d, st, sc.cfg, TOL[precision])
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("n", [2000, 6000, 12000])
+def test_large_sets_in_split_tiles(oracle, wflib, n, precision):
+    """Staged sets left uncompacted, above the LDS set: the loops take them in
+    passes, with 16, 8 and 4 lanes a particle."""
+    sc = _scenario(n, precision, 0.0)
+    sc.cfg.ns_compact_max = 256
+    st = to_oracle(oracle, sc)
+    st.nsearch(sc.cfg)
+    with to_gpu(sc, wflib) as d:
+        d.nsearch()
         _passes(d, st, sc.cfg, TOL[precision])

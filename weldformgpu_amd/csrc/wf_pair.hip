@@ -2115,15 +2115,34 @@ static void launch_timed(void (*kernel)(Fields, TileLists, typename K::Prm), dim
     hipLaunchKernelGGL(kernel, grid, block, 0, s, f, tl, p);
   }
 }
-// one pair pass over nt tiles, the neighbours staged whole (LDS) or gathered
-// (with its dispatch timestamps in g_next_launch's events when those are set)
+// One pair pass over nt tiles, the neighbours staged whole (LDS) or gathered
+// (with its dispatch timestamps in g_next_launch's events when those are set).
+//
+// A domain of few tiles leaves most of the 256 CUs idle and its passes last as
+// long as one tile's chain of loads and pairs, so a tile is dealt out to 8, 4
+// or 2 workgroups as long as they fit one a CU: each stages the whole set
+// (which costs the idle CUs nothing) and has 16, 8 or 4 lanes a particle
+// instead of 2.  Past one a CU the repeated staging costs more than the shorter
+// chain gains: Johnson-Cook step, us, with 1 / 2 / 4 / 8 workgroups a tile
+// (FP64; mixed): 17 tiles 44.4 / 38.0 / 34.0 / 33.4; 34.8 / 30.5 / 28.5 /
+// 26.3; 41 tiles 45.1 / 38.6 / 35.7 / 37.5; 35.3 / 31.2 / 29.2 / 30.0; 65
+// tiles 45.4 / 38.7 / 40.3 / 45.2; 34.9 / 30.8 / 31.4 / 31.8; 142 tiles 46.9 /
+// 48.1 / 51.5 / 60.7; 35.6 / 35.4 / 35.4 / 42.7.
 template <class K, bool LDS = true>
 static void launch_pair(hipStream_t s, int nt, const Fields& f, const TileLists& tl,
                         const typename K::Prm& p) {
-  if constexpr (LDS && HasLds<K>::on)
-    launch_timed<K>(k_pair_lds<K, 2, kTileP>, dim3(nt), dim3(2 * kTileP), s, f, tl, p);
-  else
+  if constexpr (LDS && HasLds<K>::on) {
+    constexpr int kCus = 256, kThreads = 2 * kTileP;
+    auto go = [&](auto kernel, int split) {
+      launch_timed<K>(kernel, dim3(nt * split), dim3(kThreads), s, f, tl, p);
+    };
+    if (8 * nt <= kCus) go(k_pair_lds<K, 16, kTileP / 8>, 8);
+    else if (4 * nt <= kCus) go(k_pair_lds<K, 8, kTileP / 4>, 4);
+    else if (2 * nt <= kCus) go(k_pair_lds<K, 4, kTileP / 2>, 2);
+    else go(k_pair_lds<K, 2, kTileP>, 1);
+  } else {
     launch_timed<K>(k_pair_gather<K>, dim3(nt), dim3(kTileP * K::LANES), s, f, tl, p);
+  }
 }
 
 // launch policy POL with every particle's h equal (UH) or not
