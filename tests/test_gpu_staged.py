@@ -86,3 +86,23 @@ def test_large_sets_in_split_tiles(oracle, wflib, n, precision):
     with to_gpu(sc, wflib) as d:
         d.nsearch()
         _passes(d, st, sc.cfg, TOL[precision])
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("uniform_mass", [True, False])
+def test_surface_sums_in_the_rates_pass(oracle, wflib, uniform_mass, precision):
+    """A contact step takes the free-surface sums along in the rates pass when
+    the masses are one, in a pass of its own when they are not."""
+    sc = scenarios.c4_contact(scale=0.15, r=0.25e-3, dens=12, offset=0.137)
+    sc.cfg.precision = precision
+    randomize(sc, seed=5, v_scale=0.1, shear=False)
+    if not uniform_mass:
+        sc.fields["m"][sc.n // 3] *= 1.0 + 1e-9
+    st = to_oracle(oracle, sc)
+    st.nsearch(sc.cfg)
+    st.step(sc.cfg, sc.bcs, 2)
+    with to_gpu(sc, wflib) as d:
+        d.step(2)
+        assert np.array_equal(d.get("ID"), st["ID"])
+        assert (d.get("ID") == sc.cfg.id_free_surf).sum() > 100
+        assert rel_l2(d.get("normal"), st.contact_arrays["normal"]) <= TOL[precision]

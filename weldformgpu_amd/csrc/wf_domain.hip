@@ -1706,9 +1706,19 @@ int wf_step(wf_domain* d, int n_steps) {
         if ((rc = timer_end(d, WF_K_DENS))) return rc;
       }
       dens_done = false;
+      // with one h and one mass the rates pass also sums the free-surface
+      // normals (SolverFraser.cu:233-238; the passes between read none of it)
+      const bool fuse_surf = d->cfg.contact && uh && d->uniform_m;
+      SurfaceArgs surf{};
+      if (fuse_surf) {
+        if ((rc = d->surface_init())) return rc;
+        surf = SurfaceArgs{d->cfg.id_free_surf, (double)d->n + (double)d->mesh.ne, d->totmass,
+                           d->surface_r2cut(), d->m_value};
+      }
+      const SurfaceArgs* sf = fuse_surf ? &surf : nullptr;
       timer_begin(d, true);
-      if (mx) launch_rates_mixed(d->stream, d->f, d->tl, d->solid, p.quirks, cs32, uh);
-      else launch_rates_tiled(d->stream, d->f, d->tl, d->solid, p.quirks, uh);
+      if (mx) launch_rates_mixed(d->stream, d->f, d->tl, d->solid, p.quirks, cs32, uh, sf);
+      else launch_rates_tiled(d->stream, d->f, d->tl, d->solid, p.quirks, uh, sf);
       if ((rc = timer_end(d, WF_K_RATES))) return rc;
       timer_begin(d);
       const int rec = mx ? kRec32 : kRec64;
@@ -1750,8 +1760,10 @@ int wf_step(wf_domain* d, int n_steps) {
       }
       if (d->cfg.contact) {  // SolverFraser.cu:233-257
         timer_begin(d);
-        if ((rc = d->surface_init())) return rc;
-        d->launch_surface();
+        if (!fuse_surf) {
+          if ((rc = d->surface_init())) return rc;
+          d->launch_surface();
+        }
         if (d->n_meshes > 0) {
           if (d->ts_i == 0 && (rc = d->contact_nb())) return rc;
           launch_contact_force(d->stream, d->f, d->solid, d->mesh, d->cl, d->contact_params());

@@ -253,11 +253,18 @@ struct LaunchEvents {
 };
 extern LaunchEvents g_next_launch;
 
+// what the free-surface pass needs when the rates pass takes its sums along:
+// for domains with one h and one mass m
+struct SurfaceArgs {
+  int id_free_surf;
+  double ntot, totmass, r2cut, m;
+};
+
 // FP64 pair loops (uh: every particle has the same h)
 void launch_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, int solid,
                        double dt, bool fuse, bool uh);
 void launch_rates_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        int quirks, bool uh);
+                        int quirks, bool uh, const SurfaceArgs* sf = nullptr);
 void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         double alpha, double beta, bool uh, double m_uni, double cs_uni,
                         const StatsFold& fold = {});
@@ -278,7 +285,7 @@ void launch_accel_integrate_mixed(hipStream_t s, const Fields& f, const TileList
 void launch_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n, int solid,
                        double dt, bool fuse, float cs32, bool uh);
 void launch_rates_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        int quirks, float cs32, bool uh);
+                        int quirks, float cs32, bool uh, const SurfaceArgs* sf = nullptr);
 void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         double alpha, double beta, float cs32, bool uh, bool uc, double cs_uni,
                         const StatsFold& fold = {});

@@ -23,12 +23,9 @@
 #include "wf_device.hpp"
 #include "wf_tiles.hpp"
 
-// straight-line batches (drop(), below) in the FP32 rates and FP64
-// acceleration loops: off, measured slower there (759k-particle cylinder:
-// rates 0.072 vs 0.059 ms, FP64 acceleration 0.346 vs 0.321 ms)
-#ifndef WF_DROP_RATES32
-#define WF_DROP_RATES32 0
-#endif
+// straight-line batches (drop(), below): not in the FP32 rates loop (0.072 vs
+// 0.059 ms on a 759k-particle cylinder) and off in the gathering FP64
+// acceleration loop (0.346 vs 0.321 ms)
 #ifndef WF_DROP_ACCEL64
 #define WF_DROP_ACCEL64 0
 #endif
@@ -358,23 +355,93 @@ struct DensD {
   }
 };
 
+struct NoDrop {};
+template <class Nb>
+struct DropMdj {
+  __device__ static void drop(Nb& nb) { nb.v.w = 0.0; }
+};
+
+// Free-surface sums (Geometry.cu:26-88) taken along by the rates pass, which
+// forms the same x_ij over the same lists at the same positions: the normal
+// sum_j m x_ij (every particle's mass is m) and the neighbour count, with the
+// flag decided as in the pass of its own (SurfD, SurfG).  Nothing between the
+// rates pass and the reference's surface pass reads the flags or normals.  A
+// second traversal of the lists took 157 us on a 2.74 M-particle friction-stir
+// plate in mixed precision (63 us on a 1.32 M-particle cylinder); the sums add
+// 38 us to the rates pass (8 us).
+template <class T>
+struct SurfPrm {
+  int id_free_surf;
+  double ntot, totmass;
+  T r2cut;  // > 0: lists carry a skin; count only pairs within the radius
+  T m;
+};
+// normal = n N/(M cnt); flag |normal| >= 0.25 h with at most 46 neighbours
+__device__ __forceinline__ void surface_finish(const Fields& f, int i, double nx, double ny,
+                                               double nz, int cnt, double ntot, double totmass,
+                                               int id_free_surf) {
+  const double sc = ntot / (totmass * (double)cnt);
+  nx *= sc;
+  ny *= sc;
+  nz *= sc;
+  f.nrm[0][i] = nx;
+  f.nrm[1][i] = ny;
+  f.nrm[2][i] = nz;
+  if (sqrt(nx * nx + ny * ny + nz * nz) >= 0.25 * f.h[i] && cnt <= 46 && !f.idlock[i])
+    f.ID[i] = id_free_surf;
+}
+template <bool SF>
+struct SurfSums {
+  __device__ __forceinline__ void surf_merge(const SurfSums&) {}
+  template <class T>
+  __device__ __forceinline__ void surf_add(T, T, T, T, const SurfPrm<T>&) {}
+  template <class P>
+  __device__ __forceinline__ void surf_finish(const Fields&, int, const P&) const {}
+};
+template <>
+struct SurfSums<true> {
+  double nx, ny, nz;
+  int cnt;
+  __device__ __forceinline__ void surf_merge(const SurfSums& b) {
+    nx += b.nx;
+    ny += b.ny;
+    nz += b.nz;
+    cnt += b.cnt;
+  }
+  // FP32 terms are rounded to FP32 and summed in FP64
+  template <class T>
+  __device__ __forceinline__ void surf_add(T dx, T dy, T dz, T r2, const SurfPrm<T>& p) {
+    if (p.r2cut > (T)0 && !(r2 < p.r2cut)) return;
+    const T tx = p.m * dx, ty = p.m * dy, tz = p.m * dz;
+    nx += tx;
+    ny += ty;
+    nz += tz;
+    cnt++;
+  }
+  template <class P>
+  __device__ __forceinline__ void surf_finish(const Fields& f, int i, const P& p) const {
+    surface_finish(f, i, nx, ny, nz, cnt, p.ntot, p.totmass, p.id_free_surf);
+  }
+};
+
 // B: strain rate -1/2 sum (m_j/rho_j) GK (v_ij (x) x_ij + x_ij (x) v_ij) and
 // rotation rate -1/2 sum (m_j/rho_j) GK (v_ij (x) x_ij - x_ij (x) v_ij),
 // upper triangle, xz optionally negated (InteractionAlt.cu:262-383)
-template <bool UH>
-struct RatesD {
+// SF: the free-surface sums of the same pairs as well (SurfSums)
+template <bool UH, bool SF = false>
+struct RatesD : std::conditional_t<SF, NoDrop, DropMdj<typename DensD<UH>::Nb>> {
   WF_GATHER64
   static constexpr int NBATCH = 4;
   struct Prm {
     int limit;
     double xz_sign;
+    SurfPrm<double> sf;
   };
   struct Own {
     double x, y, z, vx, vy, vz;
     HConst hc;
   };
   typedef typename DensD<UH>::Nb Nb;
-  __device__ static void drop(Nb& nb) { DensD<UH>::drop(nb); }
   WF_LDS64(3, 1)
   __device__ static void lds_put(const Fields& f, int j, const Ctx& c, double2 (&q)[3],
                                  double (&r)[1]) {
@@ -384,16 +451,17 @@ struct RatesD {
                                  double& z, Nb& nb) {
     DensD<UH>::lds_get(q, r, x, y, z, nb);
   }
-  struct Acc {
+  struct Acc : SurfSums<SF> {
     double dxx, dyy, dzz, dxy, dyz, dxz, wxy, wyz, wxz;
   };
   __device__ static void merge(Acc& a, const Acc& b) {
     a.dxx += b.dxx; a.dyy += b.dyy; a.dzz += b.dzz;
     a.dxy += b.dxy; a.dyz += b.dyz; a.dxz += b.dxz;
     a.wxy += b.wxy; a.wyz += b.wyz; a.wxz += b.wxz;
+    a.surf_merge(b);
   }
   __device__ static void init(const Fields& f, int i, bool act, Own& o, Acc& a, const Ctx&) {
-    a = Acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
+    a = Acc{};
     if (!act) return;
     o.x = f.x[0][i]; o.y = f.x[1][i]; o.z = f.x[2][i];
     o.vx = f.v[0][i]; o.vy = f.v[1][i]; o.vz = f.v[2][i];
@@ -401,9 +469,10 @@ struct RatesD {
   }
   __device__ static void load(const Fields& f, int j, Nb& nb) { DensD<UH>::load(f, j, nb); }
   __device__ static void pair(double x, double y, double z, const Nb& nb, const Own& o, Acc& a,
-                              const Prm&) {
+                              const Prm& p) {
     const double xx = o.x - x, xy = o.y - y, xz = o.z - z;
     const double r2 = xx * xx + xy * xy + xz * xz;
+    a.surf_add(xx, xy, xz, r2, p.sf);
     double rinv, h_;
     const double w = gk_pair(r2, UH ? o.hc.h : nb.h, o.hc, rinv, h_) * nb.v.w;
     const double vx = o.vx - nb.v.x, vy = o.vy - nb.v.y, vz = o.vz - nb.v.z;
@@ -426,6 +495,7 @@ struct RatesD {
     f.strrate[5][i] = -0.5 * a.dxz;
     f.rotrate[3][i] = -0.5 * a.wxy; f.rotrate[4][i] = -0.5 * a.wyz;  // diagonal stays 0
     f.rotrate[5][i] = -0.5 * p.xz_sign * a.wxz;
+    a.surf_finish(f, i, p.sf);
   }
 };
 
@@ -1457,7 +1527,8 @@ struct DensG {
 // FP32 before adding them to FP64 was as fast but doubled the plastic-strain
 // and temperature error of a 3,000-step Johnson-Cook run against FP64
 // (5.6e-5 vs 2.8e-5).
-template <bool UH>
+// SF: the free-surface sums of the same pairs as well (SurfSums)
+template <bool UH, bool SF = false>
 struct RatesG {
   WF_GATHER32
   static constexpr int NBATCH = 4;
@@ -1465,12 +1536,10 @@ struct RatesG {
     int limit;
     double xz_sign;
     float cs;
+    SurfPrm<float> sf;
   };
   typedef typename DensG<UH>::Own Own;
   typedef typename DensG<UH>::Nb Nb;
-#if WF_DROP_RATES32
-  __device__ static void drop(Nb& nb) { DensG<UH>::drop(nb); }
-#endif
   // the neighbour's {v, m/rho} is staged in LDS with its position
   typedef float4 Extra;
   __device__ static Extra extra(const Fields& f, int j) { return gat<float4>(f.v4, j); }
@@ -1493,16 +1562,17 @@ struct RatesG {
   // adding it costs 27 operations, and this loop is bound by its vector ALU:
   // on a 759k-particle cylinder 0.082 -> 0.066 ms, with the same error
   // against the FP64 rates (4.7e-7 relative L2; the FP32 factors set it)
-  struct Acc {
+  struct Acc : SurfSums<SF> {
     double xx, yy, zz, xy, yx, yz, zy, xz, zx;
   };
   __device__ static void merge(Acc& a, const Acc& b) {
     a.xx += b.xx; a.yy += b.yy; a.zz += b.zz;
     a.xy += b.xy; a.yx += b.yx; a.yz += b.yz;
     a.zy += b.zy; a.xz += b.xz; a.zx += b.zx;
+    a.surf_merge(b);
   }
   __device__ static void init(const Fields& f, int i, bool act, Own& o, Acc& a, const Ctx32& c) {
-    a = Acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
+    a = Acc{};
     if (!act) return;
     pos32(f, i, c, o.x, o.y, o.z);
     const float4 v = f.v4[i];
@@ -1510,9 +1580,10 @@ struct RatesG {
     o.hc = hconst_f(f.h32[i]);
   }
   __device__ static void pair(float x, float y, float z, const Nb& nb, const Own& o, Acc& a,
-                              const Prm&) {
+                              const Prm& p) {
     const float xx = o.x - x, xy = o.y - y, xz = o.z - z;
     const float r2 = xx * xx + xy * xy + xz * xz;
+    a.surf_add(xx, xy, xz, r2, p.sf);
     float h_;
     const float w = gk_pair_f<UH>(r2, nb.h, o.hc, h_) * nb.v.w;
     const float vx = o.vx - nb.v.x, vy = o.vy - nb.v.y, vz = o.vz - nb.v.z;
@@ -1542,6 +1613,7 @@ struct RatesG {
     f.rotrate32[3][i] = (float)(-0.5 * (xy - yx));  // the diagonal stays 0
     f.rotrate32[4][i] = (float)(-0.5 * (yz - zy));
     f.rotrate32[5][i] = (float)(-0.5 * p.xz_sign * (xz - zx));
+    a.surf_finish(f, i, p.sf);
   }
 };
 
@@ -1863,13 +1935,7 @@ struct SurfD {
   __device__ static void finish(const Fields& f, int i, bool act, const Own&, const Acc& a,
                                 const Prm& p) {
     if (!act) return;
-    const double sc = p.ntot / (p.totmass * (double)a.cnt);
-    const double nx = a.nx * sc, ny = a.ny * sc, nz = a.nz * sc;
-    f.nrm[0][i] = nx;
-    f.nrm[1][i] = ny;
-    f.nrm[2][i] = nz;
-    if (sqrt(nx * nx + ny * ny + nz * nz) >= 0.25 * f.h[i] && a.cnt <= 46 && !f.idlock[i])
-      f.ID[i] = p.id_free_surf;
+    surface_finish(f, i, a.nx, a.ny, a.nz, a.cnt, p.ntot, p.totmass, p.id_free_surf);
   }
 };
 
@@ -1926,13 +1992,8 @@ struct SurfG {
   __device__ static void finish(const Fields& f, int i, bool act, const Own&, const Acc& a,
                                 const Prm& p) {
     if (!act) return;
-    const double sc = p.ntot / (p.totmass * (double)a.cnt);
-    const double nx = a.nx.val() * sc, ny = a.ny.val() * sc, nz = a.nz.val() * sc;
-    f.nrm[0][i] = nx;
-    f.nrm[1][i] = ny;
-    f.nrm[2][i] = nz;
-    if (sqrt(nx * nx + ny * ny + nz * nz) >= 0.25 * f.h[i] && a.cnt <= 46 && !f.idlock[i])
-      f.ID[i] = p.id_free_surf;
+    surface_finish(f, i, a.nx.val(), a.ny.val(), a.nz.val(), a.cnt, p.ntot, p.totmass,
+                   p.id_free_surf);
   }
 };
 
@@ -2101,6 +2162,11 @@ using CondDensD = CondDens<CondD<UH>, DensD<UH>>;
 template <bool UH>
 using CondDensG = CondDens<CondG<UH>, DensG<UH>>;
 
+template <bool UH>
+using RatesDU = RatesD<UH>;
+template <bool UH>
+using RatesGU = RatesG<UH>;
+
 LaunchEvents g_next_launch = {nullptr, nullptr};
 
 template <class K>
@@ -2186,10 +2252,16 @@ void launch_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int 
   launch_gather<DensD>(s, f, tl, ntiles(n), uh, solid, n, dt, fuse ? 1 : 0);
 }
 void launch_rates_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        int quirks, bool uh) {
+                        int quirks, bool uh, const SurfaceArgs* sf) {
   if (solid <= 0) return;
   const double xz = (quirks & WF_Q_ROT_XZ_SIGN) ? -1.0 : 1.0;
-  launch_gather<RatesD>(s, f, tl, ntiles(solid), uh, solid, xz);
+  if (sf) {
+    typedef RatesD<true, true> K;
+    const SurfPrm<double> sp{sf->id_free_surf, sf->ntot, sf->totmass, sf->r2cut, sf->m};
+    launch_pair<K>(s, ntiles(solid), f, tl, K::Prm{solid, xz, sp});
+  } else {
+    launch_gather<RatesDU>(s, f, tl, ntiles(solid), uh, solid, xz, SurfPrm<double>{});
+  }
 }
 void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         double alpha, double beta, bool uh, double m_uni, double cs_uni,
@@ -2249,10 +2321,17 @@ void launch_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int 
   launch_gather<DensG>(s, f, tl, ntiles(n), uh, solid, n, dt, fuse ? 1 : 0, cs32);
 }
 void launch_rates_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
-                        int quirks, float cs32, bool uh) {
+                        int quirks, float cs32, bool uh, const SurfaceArgs* sf) {
   if (solid <= 0) return;
   const double xz = (quirks & WF_Q_ROT_XZ_SIGN) ? -1.0 : 1.0;
-  launch_gather<RatesG>(s, f, tl, ntiles(solid), uh, solid, xz, cs32);
+  if (sf) {
+    typedef RatesG<true, true> K;
+    const SurfPrm<float> sp{sf->id_free_surf, sf->ntot, sf->totmass, (float)sf->r2cut,
+                            (float)sf->m};
+    launch_pair<K>(s, ntiles(solid), f, tl, K::Prm{solid, xz, cs32, sp});
+  } else {
+    launch_gather<RatesGU>(s, f, tl, ntiles(solid), uh, solid, xz, cs32, SurfPrm<float>{});
+  }
 }
 void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         double alpha, double beta, float cs32, bool uh, bool uc, double cs_uni,
