@@ -177,11 +177,12 @@ typedef struct wf_config {
                             after the acceleration pass (dom_bid_type
                             AxiSymm_3D, SolverFraser.cu:229-231; set by a
                             cylindrical-grid slice, WeldFormGPU.cu:366-375) */
-  int fuse_integrate;    /* 1 (default): in contact-free, non-axisymmetric
-                            mixed-precision steps with every particle solid,
-                            the acceleration pass integrates each particle
-                            (BC + position/velocity update) as soon as its
-                            acceleration is summed; 0: a separate pass     */
+  int fuse_integrate;    /* 1 (default): in non-axisymmetric mixed-precision
+                            steps with every particle solid, the acceleration
+                            pass integrates each particle (BC + position/
+                            velocity update) as soon as its acceleration is
+                            summed (the contact pass those with contact
+                            candidates); 0: a separate pass                */
   int ns_compact_max;    /* a tile whose adjacent cells hold at most this
                             many candidates gets its staged set compacted to
                             the particles its lists reference; larger sets
@@ -356,7 +357,7 @@ enum {
                        next step's density pass + update (inside one
                        wf_step call, when no rebuild runs between)  */
   WF_K_ACCEL_INTEGRATE, /* acceleration pair loop with each particle's BC +
-                           position/velocity update (contact-free steps)  */
+                           position/velocity update                       */
   WF_K_COUNT_
 };
 /* Accumulated milliseconds and launch count of kernel id k.  Each timed

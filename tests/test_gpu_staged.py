@@ -106,3 +106,37 @@ def test_surface_sums_in_the_rates_pass(oracle, wflib, uniform_mass, precision):
         assert np.array_equal(d.get("ID"), st["ID"])
         assert (d.get("ID") == sc.cfg.id_free_surf).sum() > 100
         assert rel_l2(d.get("normal"), st.contact_arrays["normal"]) <= TOL[precision]
+
+
+@pytest.mark.parametrize("policy", [_abi.WF_REBUILD_EVERY_N, _abi.WF_REBUILD_PLASTIC_ZONE])
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+def test_contact_pass_over_the_listed_particles(oracle, wflib, precision, policy):
+    """Only particles with candidates take the contact pass: what a caller
+    left in the others' contact force and friction heat is gone after a step,
+    also when a reorder between two candidate searches moved the particles."""
+    sc = scenarios.c4_contact(scale=0.2, r=0.25e-3, dens=16, offset=0.137)
+    sc.cfg.precision = precision
+    sc.cfg.fric_heat = 1.0
+    sc.cfg.rebuild_policy = policy
+    if policy != _abi.WF_REBUILD_EVERY_N:
+        sc.cfg.ns_skin = 0.4 * sc.meta["dx"]
+    sc.meshes[0]["nodes"][:, 2] -= 0.05 * sc.meta["dx"]
+    st = to_oracle(oracle, sc)
+    st.nsearch(sc.cfg)
+    st.step(sc.cfg, sc.bcs, 7)
+    with to_gpu(sc, wflib) as d:
+        d.set("contforce", np.ones((sc.n, 3)))
+        d.set("q_friction", np.full(sc.n, 1e3))
+        d.step(2)
+        d.snapshot_positions()
+        d.nsearch()  # a reorder, two steps into the candidates' five
+        cnt, cf = d.get("cont_nb_count"), d.get("contforce")
+        assert 0 < (cnt > 0).sum() < sc.n
+        assert not cf[cnt == 0].any() and not d.get("q_friction")[cnt == 0].any()
+        d.step(5)
+        tol = 1e-9 if precision == _abi.WF_FP64 else 1e-4
+        cf = d.get("contforce")
+        assert np.abs(cf).sum() > 0
+        assert rel_l2(cf, st.contact_arrays["cf"]) <= tol
+        for k in ("u", "v", "sigma"):
+            assert rel_l2(d.get(k), st[k]) <= tol, k

@@ -160,6 +160,9 @@ struct wf_domain {
   ContactLists cl{};
   int* cl_list_alt = nullptr;  // the candidate rows of the next order (reorder)
   int* cnb_act = nullptr;  // particles needing candidates: length, then indices
+  bool act_valid = false;  // cnb_act holds every particle with candidates (not after a reorder)
+  bool cf_set = false;     // the caller wrote contact forces or friction heat
+  int contact_list();
   bool cont_built = false;
   bool surf_init = false;  // not_write_surf_ID and total mass taken
   double totmass = 0.0;
@@ -610,6 +613,21 @@ int wf_domain::contact_nb() {
                     cnb_act, ctr);
   HIPC(hipGetLastError());
   cont_built = true;
+  act_valid = true;
+  return WF_OK;
+}
+
+// What a contact pass over the listed particles needs: the list, after a
+// reorder made anew from the counts, and no contact force or friction heat
+// that the caller left on the particles without candidates
+int wf_domain::contact_list() {
+  if (!act_valid) {
+    hipLaunchKernelGGL(k_fill_i32v, dim3(1), dim3(64), 0, stream, cnb_act, 0, 1);
+    launch_contact_relist(stream, cl, solid, cnb_act);
+    act_valid = true;
+  }
+  if (cf_set) launch_contact_clear(stream, f, cl, solid);
+  cf_set = false;
   return WF_OK;
 }
 
@@ -924,6 +942,7 @@ int wf_set_field(wf_domain* d, int field, const void* host, size_t bytes) {
     for (int i = 1; i < d->n && d->uniform_cs; i++) d->uniform_cs = cv[i] == cv[0];
   }
   d->pick_arec64();
+  if (field == WF_F_CONTFORCE || field == WF_F_Q_FRICTION) d->cf_set = true;
   HIPC(hipMemcpyAsync(d->stage, host, bytes, hipMemcpyHostToDevice, d->stream));
   if (elem == 8 && d->plane(field, 0).f) {
     Planes6f planes{};
@@ -1027,6 +1046,7 @@ int wf_fill_field(wf_domain* d, int field, double value) {
     d->cs_value = value;
   }
   d->pick_arec64();
+  if (field == WF_F_CONTFORCE || field == WF_F_Q_FRICTION) d->cf_set = true;
   if (field == WF_F_X) {
     for (int c = 0; c < 3; c++) launch_fill_f64(d->stream, d->f.xs[c], value, d->n);
     d->snap_gen++;
@@ -1179,6 +1199,7 @@ int wf_nsearch_build(wf_domain* d) {
     std::swap(d->cl.list, d->cl_list_alt);
     launch_gather_i32(d->stream, d->spare_i, d->cl.count, d->gather, d->n);
     std::swap(d->cl.count, d->spare_i);
+    d->act_valid = false;
   }
   std::swap(d->perm, d->perm_tmp);
   if (pz)
@@ -1559,7 +1580,8 @@ int wf_calc_contact_nb(wf_domain* d) {
 int wf_calc_contact_forces(wf_domain* d) {
   if (!d) return fail(WF_E_ARG, "null domain");
   if (!d->cont_built) return fail(WF_E_STATE, "contact neighbours not built");
-  launch_contact_force(d->stream, d->f, d->solid, d->mesh, d->cl, d->contact_params());
+  if (int rc = d->contact_list()) return rc;
+  launch_contact_force(d->stream, d->f, d->solid, d->mesh, d->cl, d->contact_params(), d->cnb_act);
   HIPC(hipGetLastError());
   return WF_OK;
 }
@@ -1726,27 +1748,41 @@ int wf_step(wf_domain* d, int n_steps) {
       if ((rc = timer_end(d, WF_K_STRESS))) return rc;
       // the acceleration pass's first workgroup folds the stress statistics
       const StatsFold fold{d->bstats, (p.solid + kBlock - 1) / kBlock, d->ctr};
-      // Without contact forces or the axisymmetric clamp between them, the
-      // mixed acceleration pass integrates each particle as soon as its sum
-      // is done (the reference's BC + UpdatePosFraser + UpdateVel + BC,
-      // SolverFraser.cu:273-281): the new FP32 mirrors go to spare planes,
-      // swapped in after the pass.  (The FP64 pass, at lower occupancy, was
+      // The contact step's surface pass and candidates read nothing that the
+      // acceleration pass writes, so they run before it (SolverFraser.cu:
+      // 233-257 has them behind it): that pass can then leave the particles
+      // with candidates to the contact pass.
+      const bool contact = d->cfg.contact && d->n_meshes > 0;
+      if (d->cfg.contact) {
+        timer_begin(d);
+        if (!fuse_surf) {
+          if ((rc = d->surface_init())) return rc;
+          d->launch_surface();
+        }
+        if (contact && d->ts_i == 0 && (rc = d->contact_nb())) return rc;
+        if (contact && (rc = d->contact_list())) return rc;
+        if ((rc = timer_end(d, WF_K_CONTACT))) return rc;
+      }
+      // Without the axisymmetric clamp between them, the mixed acceleration
+      // pass integrates each particle as soon as its sum is done (the
+      // reference's BC + UpdatePosFraser + UpdateVel + BC,
+      // SolverFraser.cu:273-281), but for those with contact candidates, which
+      // the contact pass integrates: the new FP32 mirrors go to spare planes,
+      // swapped in after the passes.  (The FP64 pass, at lower occupancy, was
       // slower fused: 0.396 against 0.332 + 0.032 ms on a 759k-particle
       // cylinder.)
-      const bool fuse_int = mx && d->cfg.fuse_integrate && !d->cfg.axisymm &&
-                            !d->cfg.contact && d->solid == d->n;
+      const bool fuse_int =
+          mx && d->cfg.fuse_integrate && !d->cfg.axisymm && d->solid == d->n;
+      IntegrateOut out{};
       timer_begin(d, true);
       if (fuse_int) {
         // the FP32 pass reads no FP64 position, so x is updated in place
-        IntegrateOut out{};
         for (int c = 0; c < 3; c++) out.x[c] = d->f.x[c];
         out.p4 = d->p4_spare;
         out.v4 = d->f.v4_alt;
         launch_accel_integrate_mixed(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, cs32, uh,
                                      d->uniform_c(), d->cs_value, d->cfg.dt, d->bcs, d->frame,
-                                     out, fold);
-        std::swap(d->f.p4, d->p4_spare);
-        std::swap(d->f.v4, d->f.v4_alt);
+                                     out, contact ? d->cl.count : nullptr, fold);
         if ((rc = timer_end(d, WF_K_ACCEL_INTEGRATE))) return rc;
       } else {
         if (mx)
@@ -1758,17 +1794,19 @@ int wf_step(wf_domain* d, int n_steps) {
         if (d->cfg.axisymm) launch_axisymm_bc(d->stream, d->f, d->n);  // SolverFraser.cu:229-231
         if ((rc = timer_end(d, WF_K_ACCEL))) return rc;
       }
-      if (d->cfg.contact) {  // SolverFraser.cu:233-257
+      if (contact) {
         timer_begin(d);
-        if (!fuse_surf) {
-          if ((rc = d->surface_init())) return rc;
-          d->launch_surface();
-        }
-        if (d->n_meshes > 0) {
-          if (d->ts_i == 0 && (rc = d->contact_nb())) return rc;
-          launch_contact_force(d->stream, d->f, d->solid, d->mesh, d->cl, d->contact_params());
-        }
+        if (fuse_int)
+          launch_contact_force_integrate(d->stream, d->f, d->solid, d->mesh, d->cl,
+                                         d->contact_params(), d->cnb_act, d->bcs, d->frame, out);
+        else
+          launch_contact_force(d->stream, d->f, d->solid, d->mesh, d->cl, d->contact_params(),
+                               d->cnb_act);
         if ((rc = timer_end(d, WF_K_CONTACT))) return rc;
+      }
+      if (fuse_int) {
+        std::swap(d->f.p4, d->p4_spare);
+        std::swap(d->f.v4, d->f.v4_alt);
       }
       if (!d->is_yielding) {  // SolverFraser.cu:260-271, on the device-side max
         HIPC(hipMemcpyAsync(d->ctr_host, d->ctr, sizeof(Counters), hipMemcpyDeviceToHost,

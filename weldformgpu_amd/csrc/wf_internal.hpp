@@ -147,8 +147,14 @@ void launch_surface_mixed(hipStream_t s, const Fields& f, const TileLists& tl, i
 void launch_contact_nb(hipStream_t s, const Fields& f, int solid, const MeshDev& m,
                        const TriGrid& g, const int* start, const int* sorted,
                        const ContactLists& cl, int id_free_surf, int* act, Counters* ctr);
+// act: the particles with candidates (length, then indices), as
+// launch_contact_nb or launch_contact_relist (which appends to a cleared list)
+// leaves it; the contact force and friction heat of the others stay what they
+// are, zero unless set by the caller (launch_contact_clear)
+void launch_contact_relist(hipStream_t s, const ContactLists& cl, int solid, int* act);
+void launch_contact_clear(hipStream_t s, const Fields& f, const ContactLists& cl, int solid);
 void launch_contact_force(hipStream_t s, const Fields& f, int solid, const MeshDev& m,
-                          const ContactLists& cl, const ContactParams& cp);
+                          const ContactLists& cl, const ContactParams& cp, const int* act);
 // |cf_i| where ID_i == id, else 0
 void launch_contact_norm(hipStream_t s, const Fields& f, int n, int id, double* out);
 
@@ -230,6 +236,13 @@ struct IntegrateOut {
   float4 *p4, *v4;
 };
 
+// the contact forces, and each particle with candidates integrated (mixed
+// precision; the acceleration pass integrated the others)
+void launch_contact_force_integrate(hipStream_t s, const Fields& f, int solid, const MeshDev& m,
+                                    const ContactLists& cl, const ContactParams& cp,
+                                    const int* act, const BcTable& bc, const Frame32& fr,
+                                    const IntegrateOut& out);
+
 // device-side counters written by the kernels (one allocation)
 struct Counters {
   unsigned long long max_pl_strain_bits;  // max eps_p as ordered bits (eps_p >= 0)
@@ -272,13 +285,15 @@ void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int 
                        double h_conv, double dt, bool leap, bool first, bool uh);
 
 // the mixed acceleration pass with each particle's BC + position / velocity
-// update done as soon as its acceleration is summed (contact-free,
-// non-axisymmetric steps with every particle solid); the new positions and
-// FP32 mirrors go to out's planes (IntegrateOut, above)
+// update done as soon as its acceleration is summed (non-axisymmetric steps
+// with every particle solid), but for the particles with contact candidates
+// (contacts[i] > 0, may be null), which get their acceleration only; the new
+// positions and FP32 mirrors go to out's planes (IntegrateOut, above)
 void launch_accel_integrate_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                                   double alpha, double beta, float cs32, bool uh, bool uc,
                                   double cs_uni, double dt, const BcTable& bc, const Frame32& fr,
-                                  const IntegrateOut& out, const StatsFold& fold = {});
+                                  const IntegrateOut& out, const int* contacts,
+                                  const StatsFold& fold = {});
 
 // mixed precision (FP32 pair loops, FP32 terms summed in FP64)
 // uh: every particle has the same h; uc: also the same sound speed cs_uni

@@ -140,6 +140,9 @@ struct IntegratePrm {
   BcTable bc;
   Frame32 fr;
   IntegrateOut out;
+  // a particle with contact candidates (contacts[i] > 0) is left to the contact
+  // pass, which raises its acceleration first; null: none
+  const int* contacts;
 };
 
 // FP64 policies need no per-tile context
@@ -1756,9 +1759,11 @@ struct AccelG {
                                 const Prm& p) {
     if (!act) return;
     if constexpr (IT) {
-      integrate_apply<kRec32>(f, i, a.ax.val(), a.ay.val(), a.az.val(), p.ip.dt, p.ip.bc,
-                              p.ip.fr, p.ip.out, o.in);
-      return;
+      if (!p.ip.contacts || p.ip.contacts[i] == 0) {
+        integrate_apply<kRec32>(f, i, a.ax.val(), a.ay.val(), a.az.val(), p.ip.dt, p.ip.bc,
+                                p.ip.fr, p.ip.out, o.in);
+        return;
+      }
     }
     f.a[0][i] = a.ax.val();
     f.a[1][i] = a.ay.val();
@@ -2305,9 +2310,10 @@ static void accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int
 void launch_accel_integrate_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                                   double alpha, double beta, float cs32, bool uh, bool uc,
                                   double cs_uni, double dt, const BcTable& bc, const Frame32& fr,
-                                  const IntegrateOut& out, const StatsFold& fold) {
+                                  const IntegrateOut& out, const int* contacts,
+                                  const StatsFold& fold) {
   accel_mixed<true>(s, f, tl, solid, alpha, beta, cs32, uh, uc, cs_uni,
-                    IntegratePrm{dt, bc, fr, out}, fold);
+                    IntegratePrm{dt, bc, fr, out, contacts}, fold);
 }
 void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
                        double h_conv, double dt, bool leap, bool first, bool uh) {
