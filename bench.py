@@ -62,10 +62,13 @@ ALG_BYTES_FP64 = {"dens": 80, "rates": 144, "stress": 384, "accel": 144, "integr
                   "thermal": 120, "cond_dens": 200,
                   # the acceleration pass integrating its particles: both
                   # kernels' bytes less the acceleration's read back (24 B)
-                  "accel_integrate": 144 + 172 - 24}
+                  "accel_integrate": 144 + 172 - 24,
+                  # the rates pass updating the stress: the rates are not read back
+                  "rates_stress": 144 + 384 - 72}
 # mixed (FP32 pair-loop inputs and outputs), same accounting
 ALG_BYTES_MIXED = {"dens": 40, "rates": 72, "stress": 204, "accel": 72, "integrate": 184,
-                   "thermal": 60, "cond_dens": 100, "accel_integrate": 72 + 184 - 12}
+                   "thermal": 60, "cond_dens": 100, "accel_integrate": 72 + 184 - 12,
+                   "rates_stress": 72 + 204 - 36}
 
 
 def _cpu_info():

@@ -358,6 +358,8 @@ enum {
                        wf_step call, when no rebuild runs between)  */
   WF_K_ACCEL_INTEGRATE, /* acceleration pair loop with each particle's BC +
                            position/velocity update                       */
+  WF_K_RATES_STRESS, /* strain/rotation-rate pair loop with each particle's
+                        stress update (WF_K_STRESS)                    */
   WF_K_COUNT_
 };
 /* Accumulated milliseconds and launch count of kernel id k.  Each timed

@@ -1,0 +1,51 @@
+"""The rates pass that updates its particles' stress as soon as their sums are
+done, and what a call's inner steps leave unstored.
+
+The fused pass takes domains with one h, with the Newton return map those of
+64 particles a workgroup at least and 768 tiles at most.  Tolerances: three
+steps against the FP64 oracle, relative L2 <= 1e-9 (FP64: rounding of ~56
+terms a sum, grown by the steps' differences of neighbouring values) and 1e-4
+(mixed: FP32 terms).
+"""
+import numpy as np
+import pytest
+
+from weldformgpu_amd import _abi, scenarios
+
+from harness import MECH_FIELDS, randomize, rel_l2, to_gpu, to_oracle
+
+pytestmark = pytest.mark.gpu
+
+TOL = {_abi.WF_FP64: 1e-9, _abi.WF_MIXED: 1e-4}
+
+
+def _scenario(n, precision, newton, beta=0.0):
+    """The first n particles of a thermo-mechanical cylinder at yield."""
+    sc = scenarios.c3_johnson_cook(scale=0.3 if n < 20000 else 0.51)
+    for k, v in sc.fields.items():
+        sc.fields[k] = v[:n].copy()
+    sc.cfg.n_particles = sc.cfg.solid_count = n
+    sc.cfg.precision = precision
+    sc.cfg.return_map = _abi.WF_RETURN_NEWTON if newton else _abi.WF_RETURN_REFERENCE
+    randomize(sc, seed=n, v_scale=0.5)
+    sc.fields["T"] = 300.0 + np.random.default_rng(n).uniform(0.0, 50.0, n)
+    return sc
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("newton", [True, False])
+@pytest.mark.parametrize("n", [1, 129, 4097, 8192, 8193, 16384, 16385, 98304, 98305])
+def test_stress_update_in_the_rates_pass(oracle, wflib, n, newton, precision):
+    sc = _scenario(n, precision, newton)
+    st = to_oracle(oracle, sc)
+    st.nsearch(sc.cfg)
+    st.step(sc.cfg, sc.bcs, 3)
+    fused = not newton or 8192 < n <= 98304
+    with to_gpu(sc, wflib) as d:
+        d.set_timing(True)
+        d.step(3)
+        assert d.kernel_time("rates_stress")[1] == (3 if fused else 0)
+        assert d.kernel_time("stress")[1] == (0 if fused else 3)
+        for k in MECH_FIELDS:
+            if np.linalg.norm(st[k]) > 0.0:
+                assert rel_l2(d.get(k), st[k]) <= TOL[precision], k

@@ -70,7 +70,6 @@ struct wf_domain {
   Frame32 frame{};
   // return-map statistics and surrogate
   BlockStats* bstats = nullptr;
-  int nblk = 0;  // blocks of the per-particle stress kernel
   int64_t mlp_cap = 0;
   bool jc_newton = false;  // Johnson-Cook under the Newton return map
   // WF_REBUILD_PLASTIC_ZONE: positions at the last build, the trigger's
@@ -774,8 +773,10 @@ int wf_create(const wf_config* cfg, wf_domain** out) {
   }
   // return-map statistics, surrogate samples and weights
   d->jc_newton = cfg->return_map == WF_RETURN_NEWTON && cfg->mat.model == WF_MAT_JOHNSON_COOK;
-  d->nblk = (int)((d->npad + kBlock - 1) / kBlock);
-  if (!rc) rc = d->dev_alloc((void**)&d->bstats, sizeof(BlockStats) * (d->nblk + 1));
+  // an entry a workgroup of the stress pass, or of the rates pass that updates
+  // the stress: one a tile, or up to 256 for fewer tiles
+  const int nblk = std::max(256, (cfg->n_particles + kTileP - 1) / kTileP);
+  if (!rc) rc = d->dev_alloc((void**)&d->bstats, sizeof(BlockStats) * nblk);
   for (int k = 0; k < 4 && !rc; k++) rc = d->alloc_plane_f(&d->f.mlx[k]);
   if (!rc) rc = d->alloc_plane_f(&d->f.mly);
   if (!rc) rc = d->alloc_plane_i(&d->f.mlstep);
@@ -1738,16 +1739,24 @@ int wf_step(wf_domain* d, int n_steps) {
                            d->surface_r2cut(), d->m_value};
       }
       const SurfaceArgs* sf = fuse_surf ? &surf : nullptr;
-      timer_begin(d, true);
-      if (mx) launch_rates_mixed(d->stream, d->f, d->tl, d->solid, p.quirks, cs32, uh, sf);
-      else launch_rates_tiled(d->stream, d->f, d->tl, d->solid, p.quirks, uh, sf);
-      if ((rc = timer_end(d, WF_K_RATES))) return rc;
-      timer_begin(d);
       const int rec = mx ? kRec32 : kRec64;
-      launch_stress(d->stream, d->f, p, d->bstats, true, true, rec, mx, d->ret_args());
-      if ((rc = timer_end(d, WF_K_STRESS))) return rc;
+      // with one h the rates pass updates its particles' stress as well
+      int nstat = uh ? rates_stress_blocks(d->solid, d->jc_newton) : 0;
+      timer_begin(d, true);
+      if (nstat > 0) {
+        launch_rates_stress(d->stream, d->f, d->tl, mx, cs32, sf, p, d->bstats, d->ret_args());
+        if ((rc = timer_end(d, WF_K_RATES_STRESS))) return rc;
+      } else {
+        if (mx) launch_rates_mixed(d->stream, d->f, d->tl, d->solid, p.quirks, cs32, uh, sf);
+        else launch_rates_tiled(d->stream, d->f, d->tl, d->solid, p.quirks, uh, sf);
+        if ((rc = timer_end(d, WF_K_RATES))) return rc;
+        timer_begin(d);
+        launch_stress(d->stream, d->f, p, d->bstats, true, true, rec, mx, d->ret_args());
+        if ((rc = timer_end(d, WF_K_STRESS))) return rc;
+        nstat = (p.solid + kBlock - 1) / kBlock;
+      }
       // the acceleration pass's first workgroup folds the stress statistics
-      const StatsFold fold{d->bstats, (p.solid + kBlock - 1) / kBlock, d->ctr};
+      const StatsFold fold{d->bstats, nstat, d->ctr};
       // The contact step's surface pass and candidates read nothing that the
       // acceleration pass writes, so they run before it (SolverFraser.cu:
       // 233-257 has them behind it): that pass can then leave the particles

@@ -278,6 +278,15 @@ void launch_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int 
                        double dt, bool fuse, bool uh);
 void launch_rates_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         int quirks, bool uh, const SurfaceArgs* sf = nullptr);
+// the rates pass (of either precision, every particle with the same h) that
+// runs each particle's stress update too, one BlockStats a workgroup: how many
+// of those (0: this domain takes the separate passes).  Under the Newton
+// return map a workgroup has whole wavefronts of particles, because the
+// reported iteration counts are by wavefront.
+int rates_stress_blocks(int solid, bool jc_newton);
+void launch_rates_stress(hipStream_t s, const Fields& f, const TileLists& tl, bool mixed,
+                         float cs32, const SurfaceArgs* sf, const StepParams& sp, BlockStats* bs,
+                         const RetArgs& ra);
 void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         double alpha, double beta, bool uh, double m_uni, double cs_uni,
                         const StatsFold& fold = {});

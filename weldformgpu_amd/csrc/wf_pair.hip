@@ -20,7 +20,7 @@
 #include <climits>
 #include <type_traits>
 
-#include "wf_device.hpp"
+#include "wf_stress.hpp"
 #include "wf_tiles.hpp"
 
 // straight-line batches (drop(), below): not in the FP32 rates loop (0.072 vs
@@ -493,12 +493,24 @@ struct RatesD : std::conditional_t<SF, NoDrop, DropMdj<typename DensD<UH>::Nb>> 
   __device__ static void finish(const Fields& f, int i, bool act, const Own&, const Acc& a,
                                 const Prm& p) {
     if (!act) return;
-    f.strrate[0][i] = -a.dxx; f.strrate[1][i] = -a.dyy; f.strrate[2][i] = -a.dzz;
-    f.strrate[3][i] = -0.5 * a.dxy; f.strrate[4][i] = -0.5 * a.dyz;
-    f.strrate[5][i] = -0.5 * a.dxz;
-    f.rotrate[3][i] = -0.5 * a.wxy; f.rotrate[4][i] = -0.5 * a.wyz;  // diagonal stays 0
-    f.rotrate[5][i] = -0.5 * p.xz_sign * a.wxz;
+    double v[9];
+    rates9(a, p, v);
+    put9(f, i, v);
     a.surf_finish(f, i, p.sf);
+  }
+  // the strain rate (xx yy zz xy yz xz) and the rotation rate (xy yz xz; its
+  // diagonal stays 0) as they are stored
+  typedef double RT;
+  __device__ static void rates9(const Acc& a, const Prm& p, double (&v)[9]) {
+    v[0] = -a.dxx; v[1] = -a.dyy; v[2] = -a.dzz;
+    v[3] = -0.5 * a.dxy; v[4] = -0.5 * a.dyz; v[5] = -0.5 * a.dxz;
+    v[6] = -0.5 * a.wxy; v[7] = -0.5 * a.wyz; v[8] = -0.5 * p.xz_sign * a.wxz;
+  }
+  __device__ static void put9(const Fields& f, int i, const double (&v)[9]) {
+#pragma unroll
+    for (int k = 0; k < 6; k++) f.strrate[k][i] = v[k];
+#pragma unroll
+    for (int k = 0; k < 3; k++) f.rotrate[3 + k][i] = v[6 + k];
   }
 };
 
@@ -1255,8 +1267,21 @@ struct RestOf<K, std::void_t<typename K::Rest>> {
   static constexpr bool on = true;
   typedef typename K::Rest type;
 };
+// A policy may finish its particles with whole wavefronts, a thread a particle
+// (static constexpr bool TAIL = true): the sums then go through LDS, where the
+// staged set was (tail_put, by the lane that has them), and tail() runs in
+// every thread of the workgroup, the first P with a particle each.
+template <class K, class = void>
+struct TailOf {
+  static constexpr bool on = false;
+};
+template <class K>
+struct TailOf<K, std::void_t<decltype(K::TAIL)>> {
+  static constexpr bool on = true;
+};
 template <class K, int L, int P>
-__global__ __launch_bounds__(L * P) void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
+__global__ __launch_bounds__(L * P) __attribute__((amdgpu_waves_per_eu(WavesOf<K>::value)))
+void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
   constexpr int S = kTileP / P, NT = L * P, ST = K::SET;
   static_assert(L >= 2 && L <= 16 && (L & (L - 1)) == 0, "a power of two of lanes per particle");
   typedef typename K::LV LV;
@@ -1423,7 +1448,14 @@ __global__ __launch_bounds__(L * P) void k_pair_lds(Fields f, TileLists tl, type
     const typename K::Acc other = lane_value_xor(acc, m);
     K::merge(acc, other);
   }
-  if (sub == 0) K::finish(f, i, act, own, acc, prm);
+  if constexpr (TailOf<K>::on) {
+    __syncthreads();  // the staged set is read no more
+    if (sub == 0) K::template tail_put<P>(f, i, act, acc, prm, &sv[0][0], tid / L);
+    __syncthreads();
+    K::template tail<P>(f, b * P + tid, prm, &sv[0][0], b);
+  } else {
+    if (sub == 0) K::finish(f, i, act, own, acc, prm);
+  }
   if constexpr (FoldOf<K>::on) {
     if (blockIdx.x == 0 && prm.fold.nb > 0) {
       __syncthreads();  // the staged set is read no more: its LDS is scratch
@@ -1602,21 +1634,77 @@ struct RatesG {
     a.xz = __builtin_fma(ax, dz, a.xz);
     a.zx = __builtin_fma(az, dx, a.zx);
   }
-  __device__ static double val(double v) { return v; }
   __device__ static void finish(const Fields& f, int i, bool act, const Own&, const Acc& a,
                                 const Prm& p) {
     if (!act) return;
-    const double xy = val(a.xy), yx = val(a.yx), yz = val(a.yz), zy = val(a.zy);
-    const double xz = val(a.xz), zx = val(a.zx);
-    f.strrate32[0][i] = (float)-val(a.xx); f.strrate32[1][i] = (float)-val(a.yy);
-    f.strrate32[2][i] = (float)-val(a.zz);
-    f.strrate32[3][i] = (float)(-0.5 * (xy + yx));
-    f.strrate32[4][i] = (float)(-0.5 * (yz + zy));
-    f.strrate32[5][i] = (float)(-0.5 * (xz + zx));
-    f.rotrate32[3][i] = (float)(-0.5 * (xy - yx));  // the diagonal stays 0
-    f.rotrate32[4][i] = (float)(-0.5 * (yz - zy));
-    f.rotrate32[5][i] = (float)(-0.5 * p.xz_sign * (xz - zx));
+    float v[9];
+    rates9(a, p, v);
+    put9(f, i, v);
     a.surf_finish(f, i, p.sf);
+  }
+  typedef float RT;
+  __device__ static void rates9(const Acc& a, const Prm& p, float (&v)[9]) {
+    v[0] = (float)-a.xx; v[1] = (float)-a.yy; v[2] = (float)-a.zz;
+    v[3] = (float)(-0.5 * (a.xy + a.yx));
+    v[4] = (float)(-0.5 * (a.yz + a.zy));
+    v[5] = (float)(-0.5 * (a.xz + a.zx));
+    v[6] = (float)(-0.5 * (a.xy - a.yx));
+    v[7] = (float)(-0.5 * (a.yz - a.zy));
+    v[8] = (float)(-0.5 * p.xz_sign * (a.xz - a.zx));
+  }
+  __device__ static void put9(const Fields& f, int i, const float (&v)[9]) {
+#pragma unroll
+    for (int k = 0; k < 6; k++) f.strrate32[k][i] = v[k];
+#pragma unroll
+    for (int k = 0; k < 3; k++) f.rotrate32[3 + k][i] = v[6 + k];
+  }
+};
+
+// B and C in one pass: the rates pass R that runs its particles' stress update
+// (stress_particle) as soon as their sums are done, which saves a launch and
+// the rates' way through memory (rates_stress_blocks says where); a lane a
+// particle and whole wavefronts, because the surrogate's matrix instructions
+// take all 64 lanes.
+template <class R, int REC, bool S32>
+struct RatesStress : R {
+  static constexpr bool TAIL = true;
+  static constexpr int MIN_WAVES = 3;  // 160 registers of 168 (unasked: 170, two a SIMD)
+  struct Prm : R::Prm {
+    StepParams sp;
+    RetArgs ra;
+    BlockStats* bs;  // one entry a workgroup
+  };
+  typedef typename R::RT RT;
+  template <int P>
+  __device__ static void tail_put(const Fields& f, int i, bool act, const typename R::Acc& a,
+                                  const Prm& p, void* lds, int q) {
+    RT v[9];
+    R::rates9(a, p, v);
+    if (act) a.surf_finish(f, i, p.sf);
+    RT* sh = reinterpret_cast<RT*>(lds);
+#pragma unroll
+    for (int k = 0; k < 9; k++) sh[k * P + q] = v[k];
+  }
+  template <int P>
+  __device__ static void tail(const Fields& f, int i, const Prm& p, void* lds, int b) {
+    constexpr int NW = P >= 64 ? P / 64 : 1;  // wavefronts that update particles
+    BlockStats st{0ull, 0ull, 0ull, 0ull};
+    if (threadIdx.x < 64 * NW) {
+      const RT* sh = reinterpret_cast<const RT*>(lds) + threadIdx.x;
+      auto rates = [&](double (&d)[6], double (&w)[3]) {
+        RT v[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) v[k] = sh[k * P];
+        R::put9(f, i, v);
+#pragma unroll
+        for (int k = 0; k < 6; k++) d[k] = v[k];
+#pragma unroll
+        for (int k = 0; k < 3; k++) w[k] = v[6 + k];
+      };
+      stress_particle<true, true, REC, S32>(f, p.sp, p.ra, i, (int)threadIdx.x < P && i < p.limit,
+                                            rates, st);
+    }
+    stress_block_stats(st, NW, reinterpret_cast<BlockStats*>((RT*)lds + 9 * P), p.bs + b);
   }
 };
 
@@ -2199,18 +2287,23 @@ static void launch_timed(void (*kernel)(Fields, TileLists, typename K::Prm), dim
 // 26.3; 41 tiles 45.1 / 38.6 / 35.7 / 37.5; 35.3 / 31.2 / 29.2 / 30.0; 65
 // tiles 45.4 / 38.7 / 40.3 / 45.2; 34.9 / 30.8 / 31.4 / 31.8; 142 tiles 46.9 /
 // 48.1 / 51.5 / 60.7; 35.6 / 35.4 / 35.4 / 42.7.
+static int pair_split(int nt) {
+  constexpr int kCus = 256;
+  return 8 * nt <= kCus ? 8 : 4 * nt <= kCus ? 4 : 2 * nt <= kCus ? 2 : 1;
+}
 template <class K, bool LDS = true>
 static void launch_pair(hipStream_t s, int nt, const Fields& f, const TileLists& tl,
                         const typename K::Prm& p) {
   if constexpr (LDS && HasLds<K>::on) {
-    constexpr int kCus = 256, kThreads = 2 * kTileP;
-    auto go = [&](auto kernel, int split) {
+    constexpr int kThreads = 2 * kTileP;
+    const int split = pair_split(nt);
+    auto go = [&](auto kernel) {
       launch_timed<K>(kernel, dim3(nt * split), dim3(kThreads), s, f, tl, p);
     };
-    if (8 * nt <= kCus) go(k_pair_lds<K, 16, kTileP / 8>, 8);
-    else if (4 * nt <= kCus) go(k_pair_lds<K, 8, kTileP / 4>, 4);
-    else if (2 * nt <= kCus) go(k_pair_lds<K, 4, kTileP / 2>, 2);
-    else go(k_pair_lds<K, 2, kTileP>, 1);
+    if (split == 8) go(k_pair_lds<K, 16, kTileP / 8>);
+    else if (split == 4) go(k_pair_lds<K, 8, kTileP / 4>);
+    else if (split == 2) go(k_pair_lds<K, 4, kTileP / 2>);
+    else go(k_pair_lds<K, 2, kTileP>);
   } else {
     launch_timed<K>(k_pair_gather<K>, dim3(nt), dim3(kTileP * K::LANES), s, f, tl, p);
   }
@@ -2256,10 +2349,11 @@ void launch_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int 
   if (n <= 0) return;
   launch_gather<DensD>(s, f, tl, ntiles(n), uh, solid, n, dt, fuse ? 1 : 0);
 }
+static double xz_sign(int quirks) { return (quirks & WF_Q_ROT_XZ_SIGN) ? -1.0 : 1.0; }
 void launch_rates_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         int quirks, bool uh, const SurfaceArgs* sf) {
   if (solid <= 0) return;
-  const double xz = (quirks & WF_Q_ROT_XZ_SIGN) ? -1.0 : 1.0;
+  const double xz = xz_sign(quirks);
   if (sf) {
     typedef RatesD<true, true> K;
     const SurfPrm<double> sp{sf->id_free_surf, sf->ntot, sf->totmass, sf->r2cut, sf->m};
@@ -2329,7 +2423,7 @@ void launch_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int 
 void launch_rates_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                         int quirks, float cs32, bool uh, const SurfaceArgs* sf) {
   if (solid <= 0) return;
-  const double xz = (quirks & WF_Q_ROT_XZ_SIGN) ? -1.0 : 1.0;
+  const double xz = xz_sign(quirks);
   if (sf) {
     typedef RatesG<true, true> K;
     const SurfPrm<float> sp{sf->id_free_surf, sf->ntot, sf->totmass, (float)sf->r2cut,
@@ -2337,6 +2431,52 @@ void launch_rates_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int
     launch_pair<K>(s, ntiles(solid), f, tl, K::Prm{solid, xz, cs32, sp});
   } else {
     launch_gather<RatesGU>(s, f, tl, ntiles(solid), uh, solid, xz, cs32, SurfPrm<float>{});
+  }
+}
+// The Newton return map is a long dependent chain that only half of the
+// workgroup's wavefronts run, so with more workgroups than one round of three
+// a CU the separate pass, all lanes busy and three wavefronts a SIMD, hides it
+// better.  Step, us, separate -> fused: Johnson-Cook FP64 at 147 tiles 48.0 ->
+// 45.2, 736 tiles 92.9 -> 91.0, 1,489 tiles 150.8 -> 154.7, 5,931 tiles 594 ->
+// 617; mixed 34.9 -> 33.0, 60.1 -> 58.1, 94.8 -> 99.2, 351 -> 386; bilinear
+// FP64 at 16 tiles 27.5 -> 25.5, 162 tiles 42.2 -> 39.3, 1,598 tiles 152.7 ->
+// 149.1, 6,515 tiles 593.9 -> 595.2.
+int rates_stress_blocks(int solid, bool jc_newton) {
+  const int nt = ntiles(solid), split = pair_split(nt);
+  if (jc_newton && (nt > 768 || kTileP / split < 64)) return 0;
+  return nt * split;
+}
+void launch_rates_stress(hipStream_t s, const Fields& f, const TileLists& tl, bool mixed,
+                         float cs32, const SurfaceArgs* sf, const StepParams& sp, BlockStats* bs,
+                         const RetArgs& ra) {
+  const int solid = sp.solid;
+  if (solid <= 0) return;
+  const double xz = xz_sign(sp.quirks);
+  auto go = [&](auto tag, const auto& rp) {
+    typedef decltype(tag) K;
+    typename K::Prm p;
+    static_cast<std::decay_t<decltype(rp)>&>(p) = rp;
+    p.sp = sp;
+    p.ra = ra;
+    p.bs = bs;
+    launch_pair<K>(s, ntiles(solid), f, tl, p);
+  };
+  if (mixed) {
+    SurfPrm<float> sp32{};
+    if (sf) sp32 = {sf->id_free_surf, sf->ntot, sf->totmass, (float)sf->r2cut, (float)sf->m};
+    if (sf)
+      go(RatesStress<RatesG<true, true>, kRec32, true>{},
+         RatesG<true, true>::Prm{solid, xz, cs32, sp32});
+    else
+      go(RatesStress<RatesG<true>, kRec32, true>{}, RatesG<true>::Prm{solid, xz, cs32, sp32});
+  } else {
+    SurfPrm<double> sp64{};
+    if (sf) sp64 = {sf->id_free_surf, sf->ntot, sf->totmass, sf->r2cut, sf->m};
+    if (sf)
+      go(RatesStress<RatesD<true, true>, kRec64, false>{},
+         RatesD<true, true>::Prm{solid, xz, sp64});
+    else
+      go(RatesStress<RatesD<true>, kRec64, false>{}, RatesD<true>::Prm{solid, xz, sp64});
   }
 }
 void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
