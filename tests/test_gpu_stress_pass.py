@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from weldformgpu_amd import _abi, scenarios
+from weldformgpu_amd.domain import WfError
 
 from harness import MECH_FIELDS, randomize, rel_l2, to_gpu, to_oracle
 
@@ -49,3 +50,54 @@ def test_stress_update_in_the_rates_pass(oracle, wflib, n, newton, precision):
         for k in MECH_FIELDS:
             if np.linalg.norm(st[k]) > 0.0:
                 assert rel_l2(d.get(k), st[k]) <= TOL[precision], k
+
+
+FIELDS = MECH_FIELDS + ["T"]
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("contact", [False, True])
+def test_one_call_leaves_what_single_steps_leave(wflib, contact, precision):
+    """A call's inner steps store less; every field at its end is that of as
+    many single-step calls, bit for bit."""
+    runs = []
+    for calls in ([7], [1] * 7):
+        if contact:
+            sc = scenarios.c4_contact(scale=0.2, r=0.25e-3, dens=16, offset=0.137)
+            sc.cfg.precision = precision
+            randomize(sc, seed=3, v_scale=0.5)
+        else:
+            sc = _scenario(9000, precision, True)
+        with to_gpu(sc, wflib) as d:
+            for k in calls:
+                d.step(k)
+            runs.append({k: d.get(k) for k in FIELDS})
+    for k in FIELDS:
+        assert np.array_equal(runs[0][k], runs[1][k]), k
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+def test_call_that_a_rebuild_ends(wflib, precision):
+    """A particle flies off, and the rebuild at the sixth step refuses the
+    domain: the fields are those of the five steps before it."""
+    def case():
+        sc = _scenario(3000, precision, False)
+        sc.cfg.quirks &= ~_abi.WF_Q_STALE_NS_POS
+        sc.cfg.ns_min_plastic = 0.0
+        sc.fields["pl_strain"] = np.full(sc.n, 1e-3)
+        sc.fields["v"][np.flatnonzero(sc.fields["ID"] == 0)[-1]] = [0.0, 0.0, 1e13]
+        return sc
+    runs = []
+    with to_gpu(case(), wflib) as d:
+        d.nsearch()
+        with pytest.raises(WfError):
+            d.step(20)
+        assert d.stats()["step"] == 5
+        runs.append({k: d.get(k) for k in FIELDS})
+    with to_gpu(case(), wflib) as d:
+        d.nsearch()
+        for _ in range(5):
+            d.step(1)
+        runs.append({k: d.get(k) for k in FIELDS})
+    for k in FIELDS:
+        assert np.array_equal(runs[0][k], runs[1][k], equal_nan=True), k

@@ -127,9 +127,11 @@ __device__ __forceinline__ void integrate_apply(const Fields& f, int i, double a
   f.v[0][i] = v0;
   f.v[1][i] = v1;
   f.v[2][i] = v2;
-  f.a[0][i] = a0;
-  f.a[1][i] = a1;
-  f.a[2][i] = a2;
+  if (hit >= 0 || o.put_a) {
+    f.a[0][i] = a0;
+    f.a[1][i] = a1;
+    f.a[2][i] = a2;
+  }
   if (REC == kRec64) f.kv[i] = make_double4(v0, v1, v2, f.kv[i].w);
   if (REC == kRec32) {
     int cx, cy, cz;

@@ -319,6 +319,7 @@ StepParams wf_domain::params() const {
   p.alpha = cfg.alpha;
   p.beta = cfg.beta;
   p.quirks = cfg.quirks;
+  p.keep = 1;
   p.return_map = cfg.return_map;
   p.taylor_quinney = cfg.taylor_quinney;
   p.T_inf = cfg.T_inf;
@@ -1689,6 +1690,18 @@ static int rebuild_next_step(wf_domain* d, bool* out) {
   return WF_OK;
 }
 
+// Whether a step's stress pass stores the fields that only a caller reads
+// (StepParams::keep): in a call's last step, and where the call could end
+// early, at a list rebuild or a contact candidate search that refuses its
+// input.  In the others the next step overwrites them unread.
+static bool step_keeps(const wf_domain* d, bool last) {
+  if (last || d->plastic_zone()) return true;
+  if (d->cfg.contact && d->ts_i == 0) return true;
+  if (d->ts_i + 1 <= d->cfg.ns_interval - 1) return false;
+  const bool stale = (d->cfg.quirks & WF_Q_STALE_NS_POS) != 0;
+  return !(stale && d->nb_built && d->built_gen == d->snap_gen);  // a no-op rebuild
+}
+
 // Domain_d::MechFraserSolve loop body, SolverFraser.cu:164-399.  Inside one
 // call, a step's conduction pass and the next step's density pass share one
 // traversal of the neighbour lists when no rebuild runs between them (both
@@ -1704,6 +1717,7 @@ int wf_step(wf_domain* d, int n_steps) {
   bool dens_done = false;  // this step's density pass ran with the last conduction pass
   for (int s = 0; s < n_steps; s++) {
     StepParams p = d->params();
+    p.keep = step_keeps(d, s + 1 == n_steps);
     if (d->cfg.mechanics) {
       if ((rc = resolve_pz(d))) return rc;
       if (d->plastic_zone() ? (d->is_yielding && d->pz_pending)
@@ -1789,6 +1803,7 @@ int wf_step(wf_domain* d, int n_steps) {
         for (int c = 0; c < 3; c++) out.x[c] = d->f.x[c];
         out.p4 = d->p4_spare;
         out.v4 = d->f.v4_alt;
+        out.put_a = true;
         launch_accel_integrate_mixed(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, cs32, uh,
                                      d->uniform_c(), d->cs_value, d->cfg.dt, d->bcs, d->frame,
                                      out, contact ? d->cl.count : nullptr, fold);

@@ -558,9 +558,14 @@ struct AccelD {
     o.vx = f.v[0][i]; o.vy = f.v[1][i]; o.vz = f.v[2][i];
     o.di = f.rho[i]; o.Ci = f.Cs[i];
     o.hc = hconst(f.h[i]);
-    const double idi = 1.0 / (o.di * o.di);
-    o.s0 = f.sigma[0][i] * idi; o.s1 = f.sigma[1][i] * idi; o.s2 = f.sigma[2][i] * idi;
-    o.s3 = f.sigma[3][i] * idi; o.s4 = f.sigma[4][i] * idi; o.s5 = f.sigma[5][i] * idi;
+    // its own record's sigma/rho^2 (the stress pass may not have stored sigma)
+    if constexpr (UC) {
+      const double4 sa = f.arec64u[i], sb = f.arec64[i];
+      o.s0 = sa.x; o.s1 = sa.y; o.s2 = sb.x; o.s3 = sb.y; o.s4 = sb.z; o.s5 = sb.w;
+    } else {
+      const double4 sa = f.arec64[rec_at(f, i, 1)], sb = f.arec64[rec_at(f, i, 2)];
+      o.s0 = sa.x; o.s1 = sa.y; o.s2 = sa.z; o.s3 = sa.w; o.s4 = sb.x; o.s5 = sb.y;
+    }
   }
   __device__ static void load(const Fields& f, int j, Nb& nb) {
     nb.v = gat<double4, 96>(f.arec64, j);  // rec_at(f, j, 0..2)
@@ -1695,7 +1700,7 @@ struct RatesStress : R {
         RT v[9];
 #pragma unroll
         for (int k = 0; k < 9; k++) v[k] = sh[k * P];
-        R::put9(f, i, v);
+        if (p.sp.keep) R::put9(f, i, v);
 #pragma unroll
         for (int k = 0; k < 6; k++) d[k] = v[k];
 #pragma unroll
@@ -2440,7 +2445,8 @@ void launch_rates_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int
 // 45.2, 736 tiles 92.9 -> 91.0, 1,489 tiles 150.8 -> 154.7, 5,931 tiles 594 ->
 // 617; mixed 34.9 -> 33.0, 60.1 -> 58.1, 94.8 -> 99.2, 351 -> 386; bilinear
 // FP64 at 16 tiles 27.5 -> 25.5, 162 tiles 42.2 -> 39.3, 1,598 tiles 152.7 ->
-// 149.1, 6,515 tiles 593.9 -> 595.2.
+// 149.1, and with what only a caller reads unstored (StepParams::keep) 6,515
+// tiles 570.7 -> 557.5.
 int rates_stress_blocks(int solid, bool jc_newton) {
   const int nt = ntiles(solid), split = pair_split(nt);
   if (jc_newton && (nt > 768 || kTileP / split < 64)) return 0;

@@ -154,7 +154,7 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
     for (int k = 0; k < 6; k++) f.strain[k][i] = strain[k] + d6[k] * dt;
     if (FUSE_P) {
       p_i = 0.0 + (cs_i * cs_i) * (rho_i - p_i);
-      f.p[i] = p_i;
+      if (p.keep) f.p[i] = p_i;
     }
     T9 WT = {W.xx, W.yx, W.zx, W.xy, W.yy, W.zy, W.xz, W.yz, W.zz};
     T9 SRT = tmul(S, WT, qp);
@@ -177,7 +177,7 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
     esr = sqrt(0.5 * ((D.xx - D.yy) * (D.xx - D.yy) + (D.yy - D.zz) * (D.yy - D.zz) +
                       (D.zz - D.xx) * (D.zz - D.xx)) +
                3.0 * (D.xy * D.xy + D.yz * D.yz + D.zx * D.zx));
-    f.esr[i] = esr;
+    if (p.keep) f.esr[i] = esr;
     const double J2 = 0.5 * (S.xx * S.xx + 2.0 * S.xy * S.yx + 2.0 * S.xz * S.zx +
                              S.yy * S.yy + 2.0 * S.yz * S.zy + S.zz * S.zz);
     sig_trial = sqrt(3.0 * J2);
@@ -276,15 +276,17 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
     }
     f.sigma_y[i] = sigy;
     f.pl_strain[i] = ep;
-    f.sigma_eq[i] = sigeq;
+    if (p.keep) f.sigma_eq[i] = sigeq;
     f.qpl[i] = p.taylor_quinney * sigeq * dep / dt;
     const double pi = p_i;
     // sigma = -p I + S (Mechanical.cu:540); store upper triangle
     const double sg[6] = {-pi + S.xx, -pi + S.yy, -pi + S.zz, S.xy, S.yz, S.xz};
+    if (p.keep) {
 #pragma unroll
-    for (int k = 0; k < 6; k++) {
-      if (S32) f.sigma32[k][i] = (float)sg[k];
-      else f.sigma[k][i] = sg[k];
+      for (int k = 0; k < 6; k++) {
+        if (S32) f.sigma32[k][i] = (float)sg[k];
+        else f.sigma[k][i] = sg[k];
+      }
     }
     if (REC == kRec32) {  // sigma/rho^2, rho and Cs for the FP32 acceleration loop
       const double rho = rho_i, ir2 = 1.0 / (rho * rho);
