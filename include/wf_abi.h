@@ -177,8 +177,9 @@ typedef struct wf_config {
                             after the acceleration pass (dom_bid_type
                             AxiSymm_3D, SolverFraser.cu:229-231; set by a
                             cylindrical-grid slice, WeldFormGPU.cu:366-375) */
-  int fuse_integrate;    /* 1 (default): in non-axisymmetric mixed-precision
-                            steps with every particle solid, the acceleration
+  int fuse_integrate;    /* 1 (default): in non-axisymmetric steps with every
+                            particle solid (FP64: and one h, mass and sound
+                            speed), the acceleration
                             pass integrates each particle (BC + position/
                             velocity update) as soon as its acceleration is
                             summed (the contact pass those with contact

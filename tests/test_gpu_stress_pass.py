@@ -101,3 +101,42 @@ def test_call_that_a_rebuild_ends(wflib, precision):
         runs.append({k: d.get(k) for k in FIELDS})
     for k in FIELDS:
         assert np.array_equal(runs[0][k], runs[1][k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("contact", [False, True])
+@pytest.mark.parametrize("n", [3000, 9000, 17000])
+def test_fp64_integration_in_the_acceleration_pass(wflib, n, contact):
+    """FP64: each particle integrated in the acceleration pass (those with
+    contact candidates in the contact pass) against the separate pass, over
+    steps with rebuilds: the same arithmetic in the same order, so every field
+    is bit-identical.  A domain with two masses keeps the separate pass."""
+    runs = []
+    for fuse, masses in ((1, 1), (0, 1), (1, 2)):
+        if contact:
+            scale = (n / 1320424) ** (1 / 3)
+            sc = scenarios.c4_contact(scale=scale, dens=max(6, int(64 * scale)), offset=0.137)
+            randomize(sc, seed=n, v_scale=0.5)
+        else:
+            sc = _scenario(n, _abi.WF_FP64, True)
+        sc.cfg.precision = _abi.WF_FP64
+        sc.cfg.fuse_integrate = fuse
+        sc.cfg.quirks &= ~_abi.WF_Q_STALE_NS_POS
+        sc.cfg.ns_min_plastic = 0.0
+        sc.fields["pl_strain"] = np.full(sc.n, 1e-3)
+        if masses == 2:
+            sc.fields["m"] = sc.fields["m"] * np.where(np.arange(sc.n) == 5, 1.0 + 1e-6, 1.0)
+        with to_gpu(sc, wflib) as d:
+            d.set_timing(True)
+            for k in (1, 7, 3):
+                d.step(k)
+            runs.append({k: d.get(k) for k in FIELDS + (["contforce"] if contact else [])})
+            fused = fuse and masses == 1
+            assert d.kernel_time("accel_integrate")[1] == (11 if fused else 0)
+            assert d.kernel_time("integrate")[1] == (0 if fused else 11)
+            assert d.stats()["ns_builds"] >= 2
+            if contact:
+                assert (d.get("cont_nb_count") > 0).sum() > 0
+    for k in runs[0]:
+        assert np.array_equal(runs[0][k], runs[1][k]), k
+        if k != "a":  # a mass 1e-6 apart: the same physics by the other passes
+            assert rel_l2(runs[2][k], runs[0][k]) < 1e-4, k

@@ -260,9 +260,9 @@ __global__ __launch_bounds__(256) void k_contact_clear(Fields f, ContactLists cl
 // wrote zeros for every particle without candidates: 15 us on a 12,000-particle
 // plate contact, 42 and 89 us at 1.32 M and on the 2.74 M-particle friction-stir
 // plate, against 4.7 us here, and 24 and 19 us with the integration.
-// INT: the particle is then integrated as well (the acceleration pass left it
-// out), its new mirrors written to out.
-template <bool INT>
+// REC: the particle is then integrated as well (the acceleration pass left it
+// out), its new mirrors or record written to out (kRecNone: it is not).
+template <int REC>
 __global__ __launch_bounds__(64) void k_contact_list(Fields f, MeshDev m, ContactLists cl,
                                                      ContactParams cp,
                                                      const int* __restrict__ act, BcTable bc,
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(64) void k_contact_list(Fields f, MeshDev m, Contac
     const double dt = cp.dt;
     double n[3] = {}, pp = 0.0, P[3][3] = {}, ve[3] = {};
     IntegrateIn in;
-    if (INT && cnt > 0 && q == 0) integrate_load<kRec32>(f, i, in);
+    if (REC != kRecNone && cnt > 0 && q == 0) integrate_load<REC>(f, i, in);
     if (cnt > 0) {
       mi = f.m[i];
       hi = f.h[i];
@@ -363,8 +363,8 @@ __global__ __launch_bounds__(64) void k_contact_list(Fields f, MeshDev m, Contac
     if (cnt > 0 && q == 0) {
       for (int c = 0; c < 3; c++) f.cf[c][i] = cf[c];
       f.qfric[i] = qf;
-      if constexpr (INT)
-        integrate_apply<kRec32>(f, i, a[0], a[1], a[2], dt, bc, fr, out, in);
+      if constexpr (REC != kRecNone)
+        integrate_apply<REC>(f, i, a[0], a[1], a[2], dt, bc, fr, out, in);
       else
         for (int c = 0; c < 3; c++) f.a[c][i] = a[c];
     }
@@ -478,16 +478,19 @@ void launch_contact_clear(hipStream_t s, const Fields& f, const ContactLists& cl
 void launch_contact_force(hipStream_t s, const Fields& f, int solid, const MeshDev& m,
                           const ContactLists& cl, const ContactParams& cp, const int* act) {
   if (solid > 0)
-    hipLaunchKernelGGL(k_contact_list<false>, dim3(contact_blocks(solid)), dim3(64), 0, s, f, m,
+    hipLaunchKernelGGL(k_contact_list<kRecNone>, dim3(contact_blocks(solid)), dim3(64), 0, s, f, m,
                        cl, cp, act, BcTable{}, Frame32{}, IntegrateOut{});
 }
 void launch_contact_force_integrate(hipStream_t s, const Fields& f, int solid, const MeshDev& m,
                                     const ContactLists& cl, const ContactParams& cp,
                                     const int* act, const BcTable& bc, const Frame32& fr,
-                                    const IntegrateOut& out) {
-  if (solid > 0)
-    hipLaunchKernelGGL(k_contact_list<true>, dim3(contact_blocks(solid)), dim3(64), 0, s, f, m,
-                       cl, cp, act, bc, fr, out);
+                                    const IntegrateOut& out, bool mixed) {
+  if (solid <= 0) return;
+  const dim3 g(contact_blocks(solid)), b(64);
+  if (mixed)
+    hipLaunchKernelGGL(k_contact_list<kRec32>, g, b, 0, s, f, m, cl, cp, act, bc, fr, out);
+  else
+    hipLaunchKernelGGL(k_contact_list<kRec64>, g, b, 0, s, f, m, cl, cp, act, bc, fr, out);
 }
 void launch_contact_norm(hipStream_t s, const Fields& f, int n, int id, double* out) {
   hipLaunchKernelGGL(k_contact_norm, dim3(gblk(n)), dim3(256), 0, s, f, n, id, out);

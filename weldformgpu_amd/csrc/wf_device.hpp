@@ -62,9 +62,10 @@ __device__ __forceinline__ void unpack_cell(int c, int& cx, int& cy, int& cz) {
 // the acceleration pass that integrates its own particles loads it before
 // its pair loop, so that the loads are in flight while the pairs are summed.
 struct IntegrateIn {
-  double x[3], v[3];
+  double x[3], v[3], u[3];
   int id;
   float cell, vw;  // the FP32 mirrors' kept cell and m/rho (kRec32)
+  double mdj;      // the FP64 record's m/rho (kRec64)
 };
 template <int REC>
 __device__ __forceinline__ void integrate_load(const Fields& f, int i, IntegrateIn& in) {
@@ -72,7 +73,9 @@ __device__ __forceinline__ void integrate_load(const Fields& f, int i, Integrate
   for (int c = 0; c < 3; c++) {
     in.x[c] = f.x[c][i];
     in.v[c] = f.v[c][i];
+    in.u[c] = f.u[c][i];
   }
+  if (REC == kRec64) in.mdj = f.kv[i].w;
   if (REC == kRec32) {
     in.cell = f.p4[i].w;
     in.vw = f.v4[i].w;
@@ -109,9 +112,9 @@ __device__ __forceinline__ void integrate_apply(const Fields& f, int i, double a
   o.x[0][i] = x0;
   o.x[1][i] = x1;
   o.x[2][i] = x2;
-  f.u[0][i] += u0;
-  f.u[1][i] += u1;
-  f.u[2][i] += u2;
+  f.u[0][i] = in.u[0] + u0;
+  f.u[1][i] = in.u[1] + u1;
+  f.u[2][i] = in.u[2] + u2;
   v0 += a0 * dt;
   v1 += a1 * dt;
   v2 += a2 * dt;
@@ -132,7 +135,7 @@ __device__ __forceinline__ void integrate_apply(const Fields& f, int i, double a
     f.a[1][i] = a1;
     f.a[2][i] = a2;
   }
-  if (REC == kRec64) f.kv[i] = make_double4(v0, v1, v2, f.kv[i].w);
+  if (REC == kRec64) o.kv[i] = make_double4(v0, v1, v2, in.mdj);
   if (REC == kRec32) {
     int cx, cy, cz;
     unpack_cell(__float_as_int(in.cell), cx, cy, cz);  // the cell kept since the last refresh

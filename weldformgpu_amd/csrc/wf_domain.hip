@@ -1786,27 +1786,34 @@ int wf_step(wf_domain* d, int n_steps) {
         if (contact && (rc = d->contact_list())) return rc;
         if ((rc = timer_end(d, WF_K_CONTACT))) return rc;
       }
-      // Without the axisymmetric clamp between them, the mixed acceleration
-      // pass integrates each particle as soon as its sum is done (the
-      // reference's BC + UpdatePosFraser + UpdateVel + BC,
-      // SolverFraser.cu:273-281), but for those with contact candidates, which
-      // the contact pass integrates: the new FP32 mirrors go to spare planes,
-      // swapped in after the passes.  (The FP64 pass, at lower occupancy, was
-      // slower fused: 0.396 against 0.332 + 0.032 ms on a 759k-particle
-      // cylinder.)
-      const bool fuse_int =
-          mx && d->cfg.fuse_integrate && !d->cfg.axisymm && d->solid == d->n;
+      // Without the axisymmetric clamp between them, the acceleration pass
+      // integrates each particle as soon as its sum is done (the reference's
+      // BC + UpdatePosFraser + UpdateVel + BC, SolverFraser.cu:273-281), but
+      // for those with contact candidates, which the contact pass integrates:
+      // the new positions (FP64) and records go to spare planes, swapped in
+      // after the passes.  Not the FP64 pass that gathers its neighbours'
+      // records: its lower occupancy made it slower (0.396 against 0.332 +
+      // 0.032 ms on a 759k-particle cylinder).
+      const bool fuse_int = d->cfg.fuse_integrate && !d->cfg.axisymm && d->solid == d->n &&
+                            (mx || d->f.arec64u);
+      const int* contacts = contact ? d->cl.count : nullptr;
       IntegrateOut out{};
       timer_begin(d, true);
       if (fuse_int) {
-        // the FP32 pass reads no FP64 position, so x is updated in place
-        for (int c = 0; c < 3; c++) out.x[c] = d->f.x[c];
+        for (int c = 0; c < 3; c++)  // the FP32 pass reads no FP64 position: in place
+          out.x[c] = mx ? d->f.x[c] : d->spare_d[c];
         out.p4 = d->p4_spare;
         out.v4 = d->f.v4_alt;
-        out.put_a = true;
-        launch_accel_integrate_mixed(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, cs32, uh,
-                                     d->uniform_c(), d->cs_value, d->cfg.dt, d->bcs, d->frame,
-                                     out, contact ? d->cl.count : nullptr, fold);
+        out.kv = d->f.kv_alt;
+        out.put_a = p.keep;
+        if (mx)
+          launch_accel_integrate_mixed(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta, cs32, uh,
+                                       d->uniform_c(), d->cs_value, d->cfg.dt, d->bcs, d->frame,
+                                       out, contacts, fold);
+        else
+          launch_accel_integrate_tiled(d->stream, d->f, d->tl, d->solid, p.alpha, p.beta,
+                                       d->m_value, d->cs_value, d->cfg.dt, d->bcs, out, contacts,
+                                       fold);
         if ((rc = timer_end(d, WF_K_ACCEL_INTEGRATE))) return rc;
       } else {
         if (mx)
@@ -1822,15 +1829,19 @@ int wf_step(wf_domain* d, int n_steps) {
         timer_begin(d);
         if (fuse_int)
           launch_contact_force_integrate(d->stream, d->f, d->solid, d->mesh, d->cl,
-                                         d->contact_params(), d->cnb_act, d->bcs, d->frame, out);
+                                         d->contact_params(), d->cnb_act, d->bcs, d->frame, out,
+                                         mx);
         else
           launch_contact_force(d->stream, d->f, d->solid, d->mesh, d->cl, d->contact_params(),
                                d->cnb_act);
         if ((rc = timer_end(d, WF_K_CONTACT))) return rc;
       }
-      if (fuse_int) {
+      if (fuse_int && mx) {
         std::swap(d->f.p4, d->p4_spare);
         std::swap(d->f.v4, d->f.v4_alt);
+      } else if (fuse_int) {
+        for (int c = 0; c < 3; c++) std::swap(d->f.x[c], d->spare_d[c]);
+        std::swap(d->f.kv, d->f.kv_alt);
       }
       if (!d->is_yielding) {  // SolverFraser.cu:260-271, on the device-side max
         HIPC(hipMemcpyAsync(d->ctr_host, d->ctr, sizeof(Counters), hipMemcpyDeviceToHost,

@@ -234,21 +234,23 @@ struct BcTable {
 };
 
 // Where the integration writes what other threads of the same kernel may
-// still read: the new positions (x) and FP32 mirrors (p4, v4).  The
+// still read: the new positions (x), FP32 mirrors (p4, v4) and FP64 record
+// (kv).  The
 // integration kernel writes them in place; the acceleration pass that
 // integrates its own particles writes the spare planes, swapped in after.
 struct IntegrateOut {
   double* x[3];
   float4 *p4, *v4;
+  double4* kv;
   bool put_a;  // store the acceleration (else it is there already)
 };
 
-// the contact forces, and each particle with candidates integrated (mixed
-// precision; the acceleration pass integrated the others)
+// the contact forces, and each particle with candidates integrated (the
+// acceleration pass integrated the others)
 void launch_contact_force_integrate(hipStream_t s, const Fields& f, int solid, const MeshDev& m,
                                     const ContactLists& cl, const ContactParams& cp,
                                     const int* act, const BcTable& bc, const Frame32& fr,
-                                    const IntegrateOut& out);
+                                    const IntegrateOut& out, bool mixed);
 
 // device-side counters written by the kernels (one allocation)
 struct Counters {
@@ -300,11 +302,16 @@ void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int
 void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
                        double h_conv, double dt, bool leap, bool first, bool uh);
 
-// the mixed acceleration pass with each particle's BC + position / velocity
+// the acceleration pass with each particle's BC + position / velocity
 // update done as soon as its acceleration is summed (non-axisymmetric steps
-// with every particle solid), but for the particles with contact candidates
+// with every particle solid; FP64: and the records of one h, mass and sound
+// speed, f.arec64u), but for the particles with contact candidates
 // (contacts[i] > 0, may be null), which get their acceleration only; the new
-// positions and FP32 mirrors go to out's planes (IntegrateOut, above)
+// positions and records go to out's planes (IntegrateOut, above)
+void launch_accel_integrate_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
+                                  double alpha, double beta, double m_uni, double cs_uni,
+                                  double dt, const BcTable& bc, const IntegrateOut& out,
+                                  const int* contacts, const StatsFold& fold = {});
 void launch_accel_integrate_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
                                   double alpha, double beta, float cs32, bool uh, bool uc,
                                   double cs_uni, double dt, const BcTable& bc, const Frame32& fr,

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(kBlock) void k_integrate(Fields f, int n, double dt
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   // in place: each thread reads and writes only its own particle
-  const IntegrateOut o{{f.x[0], f.x[1], f.x[2]}, f.p4, f.v4, false};
+  const IntegrateOut o{{f.x[0], f.x[1], f.x[2]}, f.p4, f.v4, f.kv, false};
   integrate_particle<REC>(f, i, f.a[0][i], f.a[1][i], f.a[2][i], dt, bc, fr, o);
 }
 

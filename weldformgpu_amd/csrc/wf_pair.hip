@@ -131,10 +131,10 @@ __device__ __forceinline__ void coload_rec(const void* base, int j, int sub, uin
   }
 }
 
-// The mixed acceleration pass may integrate each particle as soon as its sum
+// The acceleration pass may integrate each particle as soon as its sum
 // is done (the step's BC + position/velocity update, integrate_apply):
-// other tiles still read the old FP32 mirrors, so the new ones go to the
-// spare planes in out, swapped in by the caller after the pass.
+// other tiles still read the old positions and records, so the new ones go to
+// the spare planes in out, swapped in by the caller after the pass.
 struct IntegratePrm {
   double dt;
   BcTable bc;
@@ -523,8 +523,9 @@ struct RatesD : std::conditional_t<SF, NoDrop, DropMdj<typename DensD<UH>::Nb>> 
 #define WF_ACCEL64_NBATCH 2
 #endif
 // BV: the beta (quadratic) viscosity term is on; UC: every particle has the
-// same mass and sound speed (and h), so a pair reads neither
-template <bool UH, bool BV = false, bool UC = false>
+// same mass and sound speed (and h), so a pair reads neither; IT: each particle
+// is integrated as soon as its sum is done (IntegratePrm)
+template <bool UH, bool BV = false, bool UC = false, bool IT = false>
 struct AccelD {
   WF_GATHER64
   static constexpr int NBATCH = WF_ACCEL64_NBATCH;
@@ -533,10 +534,13 @@ struct AccelD {
     double alpha, beta;
     StatsFold fold;  // the stress pass's statistics, folded by workgroup 0
     double m_uni, cs_uni;  // UC
+    IntegratePrm ip;       // IT
   };
+  struct NoIn {};
   struct Own {
     double x, y, z, vx, vy, vz, di, Ci, s0, s1, s2, s3, s4, s5;
     HConst hc;
+    std::conditional_t<IT, IntegrateIn, NoIn> in;
   };
   struct Nb {
     double4 v, sa, sb;  // {v, m}, sigma/rho^2 xx yy zz xy, {yz, xz, rho, Cs}
@@ -558,6 +562,7 @@ struct AccelD {
     o.vx = f.v[0][i]; o.vy = f.v[1][i]; o.vz = f.v[2][i];
     o.di = f.rho[i]; o.Ci = f.Cs[i];
     o.hc = hconst(f.h[i]);
+    if constexpr (IT) integrate_load<kRec64>(f, i, o.in);
     // its own record's sigma/rho^2 (the stress pass may not have stored sigma)
     if constexpr (UC) {
       const double4 sa = f.arec64u[i], sb = f.arec64[i];
@@ -654,9 +659,16 @@ struct AccelD {
       a.az += mxz * gx + myz * gy + mzz * gz;
     }
   }
-  __device__ static void finish(const Fields& f, int i, bool act, const Own&, const Acc& a,
-                                const Prm&) {
+  __device__ static void finish(const Fields& f, int i, bool act, const Own& o, const Acc& a,
+                                const Prm& p) {
     if (!act) return;
+    if constexpr (IT) {
+      if (!p.ip.contacts || p.ip.contacts[i] == 0) {
+        integrate_apply<kRec64>(f, i, a.ax, a.ay, a.az, p.ip.dt, p.ip.bc, p.ip.fr, p.ip.out,
+                                o.in);
+        return;
+      }
+    }
     f.a[0][i] = a.ax;
     f.a[1][i] = a.ay;
     f.a[2][i] = a.az;
@@ -2373,7 +2385,7 @@ void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int
   if (solid <= 0) return;
   auto go = [&](auto tag, auto lds) {
     typedef decltype(tag) K;
-    const typename K::Prm p{solid, alpha, beta, fold, m_uni, cs_uni};
+    const typename K::Prm p{solid, alpha, beta, fold, m_uni, cs_uni, IntegratePrm{}};
     launch_pair<K, lds()>(s, ntiles(solid), f, tl, p);
   };
   const std::true_type yes;
@@ -2384,6 +2396,19 @@ void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int
     beta != 0.0 ? go(AccelD<true, true>{}, no) : go(AccelD<true, false>{}, no);
   else
     beta != 0.0 ? go(AccelD<false, true>{}, no) : go(AccelD<false, false>{}, no);
+}
+void launch_accel_integrate_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int solid,
+                                  double alpha, double beta, double m_uni, double cs_uni,
+                                  double dt, const BcTable& bc, const IntegrateOut& out,
+                                  const int* contacts, const StatsFold& fold) {
+  if (solid <= 0) return;
+  auto go = [&](auto tag) {
+    typedef decltype(tag) K;
+    launch_pair<K>(s, ntiles(solid), f, tl,
+                   typename K::Prm{solid, alpha, beta, fold, m_uni, cs_uni,
+                                   IntegratePrm{dt, bc, Frame32{}, out, contacts}});
+  };
+  beta != 0.0 ? go(AccelD<true, true, true, true>{}) : go(AccelD<true, false, true, true>{});
 }
 // uc: every particle has the same h and sound speed cs_uni
 template <bool IT>
