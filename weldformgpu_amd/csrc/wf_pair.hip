@@ -967,18 +967,33 @@ struct WavesOf<K, std::void_t<decltype(K::MIN_WAVES)>> {
   static constexpr int value = K::MIN_WAVES;
 };
 
-// the value v holds in lane (this lane ^ m)
-template <class T>
-__device__ __forceinline__ T lane_value_xor(const T& v, int m) {
+// the value v holds in lane (this lane ^ M), M = 1, 2, 4 or 8, where the M
+// lanes of an aligned group hold the same value (a butterfly's steps): by DPP,
+// so that no trip through the LDS pipe is waited for.  quad_perm [1, 0, 3, 2]
+// and [2, 3, 0, 1], row_half_mirror (lane 7 - i of 8), row_mirror (15 - i)
+template <int M, class T>
+__device__ __forceinline__ T lane_value_xor(const T& v) {
   static_assert(sizeof(T) % 4 == 0, "whole 32-bit words");
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a row of 16 lanes");
+  constexpr int CTRL = M == 1 ? 0xB1 : M == 2 ? 0x4E : M == 4 ? 0x141 : 0x140;
   constexpr int W = sizeof(T) / 4;
   int in[W], out[W];
   __builtin_memcpy(in, &v, sizeof(T));
 #pragma unroll
-  for (int w = 0; w < W; w++) out[w] = __shfl_xor(in[w], m);
+  for (int w = 0; w < W; w++)
+    out[w] = __builtin_amdgcn_update_dpp(0, in[w], CTRL, 0xF, 0xF, false);
   T r;
   __builtin_memcpy(&r, out, sizeof(T));
   return r;
+}
+// the sums of a particle's L lanes merged, in every one of them
+template <class K, int L, int M = 1>
+__device__ __forceinline__ void merge_lanes(typename K::Acc& acc) {
+  if constexpr (M < L) {
+    const typename K::Acc other = lane_value_xor<M>(acc);
+    K::merge(acc, other);
+    merge_lanes<K, L, 2 * M>(acc);
+  }
 }
 
 // A pair functor may load its neighbour records cooperatively (static
@@ -1224,13 +1239,7 @@ void k_pair_gather(Fields f, TileLists tl, typename K::Prm prm) {
       }
     }
   }
-  if constexpr (L > 1) {
-#pragma unroll
-    for (int m = 1; m < L; m <<= 1) {
-      const typename K::Acc other = lane_value_xor(acc, m);
-      K::merge(acc, other);
-    }
-  }
+  merge_lanes<K, L>(acc);
   if (sub == 0) K::finish(f, i, act, own, acc, prm);
   if constexpr (FoldOf<K>::on) {
     if (blockIdx.x == 0 && prm.fold.nb > 0) {
@@ -1288,13 +1297,17 @@ struct RestOf<K, std::void_t<typename K::Rest>> {
 // (static constexpr bool TAIL = true): the sums then go through LDS, where the
 // staged set was (tail_put, by the lane that has them), and tail() runs in
 // every thread of the workgroup, the first P with a particle each.
+// What tail() reads of its particle may be loaded ahead of the pair loop
+// (static constexpr bool PRE = true; Pre, pre()).
 template <class K, class = void>
 struct TailOf {
-  static constexpr bool on = false;
+  static constexpr bool on = false, pre = false;
+  typedef int type;
 };
 template <class K>
 struct TailOf<K, std::void_t<decltype(K::TAIL)>> {
-  static constexpr bool on = true;
+  static constexpr bool on = true, pre = K::PRE;
+  typedef typename K::Pre type;
 };
 template <class K, int L, int P>
 __global__ __launch_bounds__(L * P) __attribute__((amdgpu_waves_per_eu(WavesOf<K>::value)))
@@ -1323,6 +1336,9 @@ void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
   typename K::Own own;
   typename K::Acc acc;
   K::init(f, i, act, own, acc, cx);
+  typename TailOf<K>::type pre;
+  if constexpr (TailOf<K>::pre)
+    if (tid < P && b * P + tid < prm.limit) K::pre(f, b * P + tid, pre);
   // SU neighbours per thread at a time: their indices, then everything the
   // pairs read of them, then the LDS writes
   auto stage = [&](int c0, int m) {
@@ -1460,16 +1476,12 @@ void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
       }
     }
   }
-#pragma unroll
-  for (int m = 1; m < L; m <<= 1) {
-    const typename K::Acc other = lane_value_xor(acc, m);
-    K::merge(acc, other);
-  }
+  merge_lanes<K, L>(acc);
   if constexpr (TailOf<K>::on) {
     __syncthreads();  // the staged set is read no more
     if (sub == 0) K::template tail_put<P>(f, i, act, acc, prm, &sv[0][0], tid / L);
     __syncthreads();
-    K::template tail<P>(f, b * P + tid, prm, &sv[0][0], b);
+    K::template tail<P>(f, b * P + tid, prm, &sv[0][0], b, pre);
   } else {
     if (sub == 0) K::finish(f, i, act, own, acc, prm);
   }
@@ -1682,10 +1694,20 @@ struct RatesG {
 // the rates' way through memory (rates_stress_blocks says where); a lane a
 // particle and whole wavefronts, because the surrogate's matrix instructions
 // take all 64 lanes.
-template <class R, int REC, bool S32>
+// AHEAD: with a tile dealt out to several workgroups, at most one a CU, there
+// are registers to load what the update reads before the pair loop.  FP64
+// step, us: 2,000 bilinear particles 22.2 -> 21.5, 8,272 Johnson-Cook 33.2 ->
+// 33.0; not with whole tiles (20,640: 35.7 -> 36.0) nor in mixed precision
+// (8,272: 27.0 -> 27.5).
+template <class R, int REC, bool S32, bool AHEAD>
 struct RatesStress : R {
-  static constexpr bool TAIL = true;
-  static constexpr int MIN_WAVES = 3;  // 160 registers of 168 (unasked: 170, two a SIMD)
+  static constexpr bool TAIL = true, PRE = AHEAD;
+  typedef StressIn Pre;
+  __device__ static void pre(const Fields& f, int i, Pre& in) {
+    stress_load<true, true, S32>(f, i, in);
+  }
+  // 160 registers of 168 (unasked: 170, two a SIMD)
+  static constexpr int MIN_WAVES = AHEAD ? 1 : 3;
   struct Prm : R::Prm {
     StepParams sp;
     RetArgs ra;
@@ -1703,7 +1725,7 @@ struct RatesStress : R {
     for (int k = 0; k < 9; k++) sh[k * P + q] = v[k];
   }
   template <int P>
-  __device__ static void tail(const Fields& f, int i, const Prm& p, void* lds, int b) {
+  __device__ static void tail(const Fields& f, int i, const Prm& p, void* lds, int b, Pre& in) {
     constexpr int NW = P >= 64 ? P / 64 : 1;  // wavefronts that update particles
     BlockStats st{0ull, 0ull, 0ull, 0ull};
     if (threadIdx.x < 64 * NW) {
@@ -1718,8 +1740,9 @@ struct RatesStress : R {
 #pragma unroll
         for (int k = 0; k < 3; k++) w[k] = v[6 + k];
       };
-      stress_particle<true, true, REC, S32>(f, p.sp, p.ra, i, (int)threadIdx.x < P && i < p.limit,
-                                            rates, st);
+      const bool active = (int)threadIdx.x < P && i < p.limit;
+      if (!AHEAD && active) pre(f, i, in);
+      stress_particle<true, true, REC, S32>(f, p.sp, p.ra, i, active, in, rates, st);
     }
     stress_block_stats(st, NW, reinterpret_cast<BlockStats*>((RT*)lds + 9 * P), p.bs + b);
   }
@@ -2492,22 +2515,27 @@ void launch_rates_stress(hipStream_t s, const Fields& f, const TileLists& tl, bo
     p.bs = bs;
     launch_pair<K>(s, ntiles(solid), f, tl, p);
   };
+  auto pick = [&](auto rates, auto mx, const auto& rp) {
+    typedef decltype(rates) R;
+    if constexpr (mx()) {
+      go(RatesStress<R, kRec32, true, false>{}, rp);
+    } else {
+      if (pair_split(ntiles(solid)) > 1) go(RatesStress<R, kRec64, false, true>{}, rp);
+      else go(RatesStress<R, kRec64, false, false>{}, rp);
+    }
+  };
+  const std::true_type yes;
+  const std::false_type no;
   if (mixed) {
     SurfPrm<float> sp32{};
     if (sf) sp32 = {sf->id_free_surf, sf->ntot, sf->totmass, (float)sf->r2cut, (float)sf->m};
-    if (sf)
-      go(RatesStress<RatesG<true, true>, kRec32, true>{},
-         RatesG<true, true>::Prm{solid, xz, cs32, sp32});
-    else
-      go(RatesStress<RatesG<true>, kRec32, true>{}, RatesG<true>::Prm{solid, xz, cs32, sp32});
+    if (sf) pick(RatesG<true, true>{}, yes, RatesG<true, true>::Prm{solid, xz, cs32, sp32});
+    else pick(RatesG<true>{}, yes, RatesG<true>::Prm{solid, xz, cs32, sp32});
   } else {
     SurfPrm<double> sp64{};
     if (sf) sp64 = {sf->id_free_surf, sf->ntot, sf->totmass, sf->r2cut, sf->m};
-    if (sf)
-      go(RatesStress<RatesD<true, true>, kRec64, false>{},
-         RatesD<true, true>::Prm{solid, xz, sp64});
-    else
-      go(RatesStress<RatesD<true>, kRec64, false>{}, RatesD<true>::Prm{solid, xz, sp64});
+    if (sf) pick(RatesD<true, true>{}, no, RatesD<true, true>::Prm{solid, xz, sp64});
+    else pick(RatesD<true>{}, no, RatesD<true>::Prm{solid, xz, sp64});
   }
 }
 void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int solid,

@@ -85,6 +85,35 @@ __device__ __forceinline__ double jc_newton(const MatParams& mp, double s_trial,
   return g;
 }
 
+// What the stress update reads of its particle, so that a pass may load it
+// ahead.  Everything is read before the update's first store: the stores
+// could alias the fields, so a read behind one waits for its own trip to
+// memory.  Eleven trips in a row before, the strain's six among them: a
+// 759k-particle Johnson-Cook step went from 601 to 594 us (FP64) and from
+// 361 to 351 us (mixed).
+struct StressIn {
+  double rho, cs, p, G, T, sigma_y, ep, m, eint;  // p: rho0 with FUSE_P
+  double strain[6], s[6];
+};
+template <bool FUSE_P, bool ENERGY, bool S32>
+__device__ __forceinline__ void stress_load(const Fields& f, int i, StressIn& in) {
+  in.rho = f.rho[i];
+  in.cs = f.Cs[i];
+  in.p = FUSE_P ? f.rho0[i] : f.p[i];
+  in.G = f.G[i];
+  in.T = f.T[i];
+  in.sigma_y = f.sigma_y[i];
+  in.ep = f.pl_strain[i];
+#pragma unroll
+  for (int k = 0; k < 6; k++) in.strain[k] = f.strain[k][i];
+  if (ENERGY) {
+    in.m = f.m[i];
+    in.eint = f.eint[i];
+  }
+#pragma unroll
+  for (int k = 0; k < 6; k++) in.s[k] = S32 ? (double)f.ss32[k][i] : f.ss[k][i];
+}
+
 // ---------------------------------------------------------------------------
 // C: Jaumann stress update + return map, StressStrainOne (Mechanical.cu:458-554),
 // optionally with the pressure (FUSE_P), the per-particle internal-energy
@@ -106,42 +135,35 @@ __device__ __forceinline__ double jc_newton(const MatParams& mp, double s_trial,
 // 64 lanes); lanes without a particle pass active = false.  rates(d, w) gives
 // the particle's strain rate (xx yy zz xy yz xz) and rotation rate (xy yz xz);
 // st receives its share of the block statistics (wave_iters: unset).
+// in: what stress_load read of it.
 template <bool FUSE_P, bool ENERGY, int REC, bool S32, class RATES>
 __device__ __forceinline__ void stress_particle(const Fields& f, const StepParams& p,
                                                 const RetArgs& ra, int i, bool active,
-                                                const RATES& rates, BlockStats& st) {
+                                                const StressIn& in, const RATES& rates,
+                                                BlockStats& st) {
   st = BlockStats{0ull, 0ull, 0ull, 0ull};
   const MatParams& mp = p.mat;
   const double dt = p.dt;
   T9 S{}, D{};
-  double G = 0.0, sig_trial = 0.0, sigy = 0.0, ep = 0.0, sigeq = 0.0, dep = 0.0, scale = 1.0;
+  double sig_trial = 0.0, sigy = 0.0, ep = 0.0, sigeq = 0.0, dep = 0.0, scale = 1.0;
   double esr = 0.0, T = 0.0, rt = 1.0, gmax = 0.0;
-  // Everything of the particle is read before the first store: the stores
-  // could alias the fields, so a read behind one waits for its own trip to
-  // memory.  Eleven trips in a row before, the strain's six among them: a
-  // 759k-particle Johnson-Cook step went from 601 to 594 us (FP64) and from
-  // 361 to 351 us (mixed).
-  double rho_i = 0.0, cs_i = 0.0, p_i = 0.0, m_i = 0.0, eint = 0.0;
+  double G = 0.0, rho_i = 0.0, cs_i = 0.0, p_i = 0.0, m_i = 0.0, eint = 0.0;
   bool newton = false;  // a yielding Johnson-Cook particle under the Newton return map
   if (active) {
     const bool qp = (p.quirks & WF_Q_TENSOR_PRODUCT) != 0;
-    rho_i = f.rho[i];
-    cs_i = f.Cs[i];
-    p_i = FUSE_P ? f.rho0[i] : f.p[i];
-    G = f.G[i];
-    T = f.T[i];
-    sigy = f.sigma_y[i];
-    ep = f.pl_strain[i];
-    double strain[6];
-#pragma unroll
-    for (int k = 0; k < 6; k++) strain[k] = f.strain[k][i];
+    rho_i = in.rho;
+    cs_i = in.cs;
+    p_i = in.p;
+    G = in.G;
+    T = in.T;
+    sigy = in.sigma_y;
+    ep = in.ep;
     if (ENERGY) {
-      m_i = f.m[i];
-      eint = f.eint[i];
+      m_i = in.m;
+      eint = in.eint;
     }
-    auto ss = [&](int k) { return S32 ? (double)f.ss32[k][i] : f.ss[k][i]; };
-    S.xx = ss(0); S.yy = ss(1); S.zz = ss(2);
-    S.xy = S.yx = ss(3); S.yz = S.zy = ss(4); S.xz = S.zx = ss(5);
+    S.xx = in.s[0]; S.yy = in.s[1]; S.zz = in.s[2];
+    S.xy = S.yx = in.s[3]; S.yz = S.zy = in.s[4]; S.xz = S.zx = in.s[5];
     double d6[6], w3[3];
     rates(d6, w3);
     D.xx = d6[0]; D.yy = d6[1]; D.zz = d6[2];
@@ -151,7 +173,7 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
     W.xy = w3[0]; W.yz = w3[1]; W.xz = w3[2];
     W.yx = -W.xy; W.zy = -W.yz; W.zx = -W.xz;
 #pragma unroll
-    for (int k = 0; k < 6; k++) f.strain[k][i] = strain[k] + d6[k] * dt;
+    for (int k = 0; k < 6; k++) f.strain[k][i] = in.strain[k] + d6[k] * dt;
     if (FUSE_P) {
       p_i = 0.0 + (cs_i * cs_i) * (rho_i - p_i);
       if (p.keep) f.p[i] = p_i;
