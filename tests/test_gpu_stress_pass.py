@@ -140,3 +140,24 @@ def test_fp64_integration_in_the_acceleration_pass(wflib, n, contact):
         assert np.array_equal(runs[0][k], runs[1][k]), k
         if k != "a":  # a mass 1e-6 apart: the same physics by the other passes
             assert rel_l2(runs[2][k], runs[0][k]) < 1e-4, k
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("field", ["G", "rho0", "Cs", "m"])
+def test_constants_that_differ(oracle, wflib, field, precision):
+    """With one rest density, shear modulus, mass and sound speed the stress
+    update reads none of the four planes; a particle apart brings them back."""
+    sc = _scenario(9000, precision, True)
+    uniform = sc.fields[field].copy()
+    sc.fields[field][4321] *= 1.01
+    st = to_oracle(oracle, sc)
+    st.nsearch(sc.cfg)
+    st.step(sc.cfg, sc.bcs, 2)
+    apart = sc.fields[field].copy()
+    sc.fields[field] = uniform
+    with to_gpu(sc, wflib) as d:
+        d.set(field, apart)
+        d.step(2)
+        for k in MECH_FIELDS:
+            if np.linalg.norm(st[k]) > 0.0:
+                assert rel_l2(d.get(k), st[k]) <= TOL[precision], k

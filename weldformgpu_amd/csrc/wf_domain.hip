@@ -144,6 +144,8 @@ struct wf_domain {
   double m_value = 0.0;      // surface pass skips the neighbour-mass gather)
   bool uniform_cs = true;    // and the same sound speed cs_value
   double cs_value = 0.0;
+  bool uniform_G = true, uniform_rho0 = true;  // and shear modulus, rest density
+  double G_value = 0.0, rho0_value = 0.0;
   // the FP64 acceleration record's layout (Fields::arec64u), after a change
   // of h, m or Cs; the records are then rewritten before the next pass
   bool uniform_c() const { return uniform_h && uniform_cs; }
@@ -386,6 +388,11 @@ StepParams wf_domain::params() const {
   p.beta = cfg.beta;
   p.quirks = cfg.quirks;
   p.keep = 1;
+  p.uniform = uniform_G && uniform_rho0 && uniform_m && uniform_cs;
+  p.rho0 = rho0_value;
+  p.G = G_value;
+  p.m = m_value;
+  p.Cs = cs_value;
   p.return_map = cfg.return_map;
   p.taylor_quinney = cfg.taylor_quinney;
   p.T_inf = cfg.T_inf;
@@ -1008,18 +1015,17 @@ int wf_set_field(wf_domain* d, int field, const void* host, size_t bytes) {
     d->uniform_h = true;
     for (int i = 1; i < d->n && d->uniform_h; i++) d->uniform_h = hv[i] == hv[0];
   }
-  if (field == WF_F_M) {
-    const double* mv = (const double*)host;
-    d->uniform_m = true;
-    d->m_value = mv[0];
-    for (int i = 1; i < d->n && d->uniform_m; i++) d->uniform_m = mv[i] == mv[0];
-  }
-  if (field == WF_F_CS) {
-    const double* cv = (const double*)host;
-    d->uniform_cs = true;
-    d->cs_value = cv[0];
-    for (int i = 1; i < d->n && d->uniform_cs; i++) d->uniform_cs = cv[i] == cv[0];
-  }
+  // whether every particle has one value, and which
+  auto uniform = [&](bool& on, double& value) {
+    const double* v = (const double*)host;
+    on = true;
+    value = v[0];
+    for (int i = 1; i < d->n && on; i++) on = v[i] == v[0];
+  };
+  if (field == WF_F_M) uniform(d->uniform_m, d->m_value);
+  if (field == WF_F_CS) uniform(d->uniform_cs, d->cs_value);
+  if (field == WF_F_G) uniform(d->uniform_G, d->G_value);
+  if (field == WF_F_RHO0) uniform(d->uniform_rho0, d->rho0_value);
   d->pick_arec64();
   if (field == WF_F_CONTFORCE || field == WF_F_Q_FRICTION) d->cf_set = true;
   HIPC(hipMemcpyAsync(d->stage, host, bytes, hipMemcpyHostToDevice, d->stream));
@@ -1121,6 +1127,14 @@ int wf_fill_field(wf_domain* d, int field, double value) {
   if (field == WF_F_CS) {
     d->uniform_cs = true;
     d->cs_value = value;
+  }
+  if (field == WF_F_G) {
+    d->uniform_G = true;
+    d->G_value = value;
+  }
+  if (field == WF_F_RHO0) {
+    d->uniform_rho0 = true;
+    d->rho0_value = value;
   }
   d->pick_arec64();
   if (field == WF_F_CONTFORCE || field == WF_F_Q_FRICTION) d->cf_set = true;
@@ -1781,10 +1795,11 @@ static bool yield_asked(const wf_domain* d, bool last) {
 // (StepParams::keep): in a call's last step, and where the call could end
 // early, at a list rebuild or a contact candidate search that refuses its
 // input.  In the others the next step overwrites them unread.
-static bool step_keeps(const wf_domain* d, bool last) {
+// ts_i: the step's count since the last due rebuild.
+static bool step_keeps(const wf_domain* d, bool last, int ts_i) {
   if (last || d->plastic_zone()) return true;
-  if (d->cfg.contact && d->ts_i == 0) return true;
-  if (d->ts_i + 1 <= d->cfg.ns_interval - 1) return false;
+  if (d->cfg.contact && ts_i == 0) return true;
+  if (ts_i + 1 <= d->cfg.ns_interval - 1) return false;
   const bool stale = (d->cfg.quirks & WF_Q_STALE_NS_POS) != 0;
   return !(stale && d->nb_built && d->built_gen == d->snap_gen);  // a no-op rebuild
 }
@@ -1804,7 +1819,9 @@ int wf_step(wf_domain* d, int n_steps) {
   bool dens_done = false;  // this step's density pass ran with the last conduction pass
   for (int s = 0; s < n_steps; s++) {
     StepParams p = d->params();
-    p.keep = step_keeps(d, s + 1 == n_steps);
+    p.keep = step_keeps(d, s + 1 == n_steps, d->ts_i);
+    const bool keep_next = step_keeps(d, s + 2 >= n_steps,
+                                      d->ts_i + 1 > d->cfg.ns_interval - 1 ? 0 : d->ts_i + 1);
     if (d->cfg.mechanics) {
       if ((rc = resolve_pz(d))) return rc;
       if (d->plastic_zone() ? (d->is_yielding && d->pz_pending)
@@ -1970,16 +1987,18 @@ int wf_step(wf_domain* d, int n_steps) {
       timer_begin(d, true);
       if (fuse && d->mixed) {
         launch_cond_dens_mixed(d->stream, d->f, d->tl, d->n, d->solid, p.T_inf, p.h_conv, p.dt,
-                               true, d->isfirst_step, d->frame.cs32, d->uniform_h, pz_d2, skin2);
+                               true, d->isfirst_step, d->frame.cs32, d->uniform_h, pz_d2, skin2,
+                               p.keep, keep_next);
       } else if (fuse) {
         launch_cond_dens_tiled(d->stream, d->f, d->tl, d->n, d->solid, p.T_inf, p.h_conv,
-                               p.dt, true, d->isfirst_step, d->uniform_h, pz_d2, skin2);
+                               p.dt, true, d->isfirst_step, d->uniform_h, pz_d2, skin2, p.keep,
+                               keep_next);
       } else if (d->mixed) {
         launch_cond_mixed(d->stream, d->f, d->tl, d->n, p.T_inf, p.h_conv, p.dt, true,
-                          d->isfirst_step, d->frame.cs32, d->uniform_h);
+                          d->isfirst_step, d->frame.cs32, d->uniform_h, p.keep);
       } else {
         launch_cond_tiled(d->stream, d->f, d->tl, d->n, p.T_inf, p.h_conv, p.dt, true,
-                          d->isfirst_step, d->uniform_h);
+                          d->isfirst_step, d->uniform_h, p.keep);
       }
       if (d->mixed) std::swap(d->f.tk4, d->f.tk4_alt);
       else std::swap(d->f.tk64, d->f.tk64_alt);

@@ -218,12 +218,17 @@ struct StepParams {
   double T_inf, h_conv;
   double newton_tol;
   int newton_max_iter;
-  // the stress pass stores what only a caller reads (pressure, sigma,
-  // sigma_eq, effective strain rate; the rates pass that runs it its rates):
+  // the passes store what only a caller reads (pressure, sigma, sigma_eq,
+  // effective strain rate, drho, dT/dt, T_b, the integrated acceleration; the
+  // rates pass that updates the stress its rates):
   // 0 in the steps of a call whose successor overwrites all of it.  They are
   // 72 of the pass's 504 bytes a particle (FP64; 48 of 350 mixed): Johnson-Cook
   // step at 759k particles 594 -> 572 us, mixed 351 -> 344
   int keep;
+  // every particle has this rest density, shear modulus, mass and sound speed:
+  // the stress update reads none of the four planes
+  int uniform;
+  double rho0, G, m, Cs;
   MatParams mat;
 };
 
@@ -300,7 +305,8 @@ void launch_accel_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int
                         double alpha, double beta, bool uh, double m_uni, double cs_uni,
                         const StatsFold& fold = {});
 void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
-                       double h_conv, double dt, bool leap, bool first, bool uh);
+                       double h_conv, double dt, bool leap, bool first, bool uh,
+                       bool keep = true);
 
 // the acceleration pass with each particle's BC + position / velocity
 // update done as soon as its acceleration is summed (non-axisymmetric steps
@@ -328,19 +334,21 @@ void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int
                         double alpha, double beta, float cs32, bool uh, bool uc, double cs_uni,
                         const StatsFold& fold = {});
 void launch_cond_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
-                       double h_conv, double dt, bool leap, bool first, float cs32, bool uh);
+                       double h_conv, double dt, bool leap, bool first, float cs32, bool uh,
+                       bool keep = true);
 // conduction of this step fused with the density pass (+ update) of the
 // next; with pz_d2 (device, FP64 bits of the plastic-zone trigger's largest
 // squared hot displacement) the density half writes nothing when
-// 4 * d2 > pz_skin2, the host's own test for a rebuild at the next step
+// 4 * d2 > pz_skin2, the host's own test for a rebuild at the next step;
+// keep, keep_next: StepParams::keep of the two steps
 void launch_cond_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n,
                             int solid, double T_inf, double h_conv, double dt, bool leap,
                             bool first, bool uh, const unsigned long long* pz_d2,
-                            double pz_skin2);
+                            double pz_skin2, bool keep, bool keep_next);
 void launch_cond_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n,
                             int solid, double T_inf, double h_conv, double dt, bool leap,
                             bool first, float cs32, bool uh, const unsigned long long* pz_d2,
-                            double pz_skin2);
+                            double pz_skin2, bool keep, bool keep_next);
 // refresh every FP32 mirror / FP64 record from the FP64 state (after uploads
 // and rebuilds)
 void launch_mirror32(hipStream_t s, const Fields& f, int n, const Frame32& fr);

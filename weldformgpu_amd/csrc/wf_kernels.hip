@@ -36,7 +36,7 @@ __global__ __launch_bounds__(kBlock) void k_stress(Fields f, StepParams p, Block
     for (int k = 0; k < 3; k++) w[k] = S32 ? (double)f.rotrate32[3 + k][i] : f.rotrate[3 + k][i];
   };
   StressIn in;
-  if (i < p.solid) stress_load<FUSE_P, ENERGY, S32>(f, i, in);
+  if (i < p.solid) stress_load<FUSE_P, ENERGY, S32>(f, p, i, in);
   BlockStats st;
   stress_particle<FUSE_P, ENERGY, REC, S32>(f, p, ra, i, i < p.solid, in, rates, st);
   stress_block_stats(st, kBlock / 64, wst, bs + blockIdx.x);

@@ -275,6 +275,7 @@ struct DensD {
     double dt;
     int fuse;
     int mdj_alt;  // write m/rho into the next conduction record (fused with conduction)
+    int skip;     // drho is overwritten unread (StepParams::keep): don't store it
   };
   struct Own {
     double x, y, z, vx, vy, vz, rho, m;
@@ -343,7 +344,7 @@ struct DensD {
                                 const Prm& p) {
     if (act) {
       const double drho = o.rho * a.s;
-      f.drho[i] = drho;
+      if (!p.skip) f.drho[i] = drho;
       if (p.fuse) {
         const double rn = o.rho + p.dt * drho;
         f.rho_alt[i] = rn;
@@ -718,6 +719,7 @@ struct CondD {
     int limit;
     double T_inf, h_conv, dt;
     int leap, first;
+    int skip;  // dT/dt and T_b are overwritten unread (StepParams::keep)
   };
   struct Own {
     double x, y, z, k, T, mdj;
@@ -788,7 +790,7 @@ struct CondD {
                                 const Prm& p) {
     if (!act) return;
     const double acc = cond_rate(f, i, a.q, o.T, p, o.in);
-    f.dTdt[i] = acc;
+    if (!p.skip) f.dTdt[i] = acc;
     if (p.leap) {
       double Tn;
       if (p.first) {
@@ -796,7 +798,7 @@ struct CondD {
         Tn = o.T;
       } else {
         const double ta = o.in.ta;
-        f.Tb[i] = ta;
+        if (!p.skip) f.Tb[i] = ta;
         double tan = ta + acc * p.dt;
         f.Ta[i] = tan;
         Tn = (tan + ta) / 2.;
@@ -1338,7 +1340,7 @@ void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
   K::init(f, i, act, own, acc, cx);
   typename TailOf<K>::type pre;
   if constexpr (TailOf<K>::pre)
-    if (tid < P && b * P + tid < prm.limit) K::pre(f, b * P + tid, pre);
+    if (tid < P && b * P + tid < prm.limit) K::pre(f, prm, b * P + tid, pre);
   // SU neighbours per thread at a time: their indices, then everything the
   // pairs read of them, then the LDS writes
   auto stage = [&](int c0, int m) {
@@ -1505,6 +1507,7 @@ struct DensG {
     int fuse;
     float cs;
     int mdj_alt;  // write m/rho into the next conduction record (fused with conduction)
+    int skip;     // drho is overwritten unread (StepParams::keep): don't store it
   };
   struct Own {
     float x, y, z, vx, vy, vz;
@@ -1567,7 +1570,7 @@ struct DensG {
     if (act) {
       const double rho = o.rho;
       const double drho = rho * a.val();
-      f.drho[i] = drho;
+      if (!p.skip) f.drho[i] = drho;
       if (p.fuse) {
         const double rn = rho + p.dt * drho;
         f.rho_alt[i] = rn;
@@ -1703,9 +1706,6 @@ template <class R, int REC, bool S32, bool AHEAD>
 struct RatesStress : R {
   static constexpr bool TAIL = true, PRE = AHEAD;
   typedef StressIn Pre;
-  __device__ static void pre(const Fields& f, int i, Pre& in) {
-    stress_load<true, true, S32>(f, i, in);
-  }
   // 160 registers of 168 (unasked: 170, two a SIMD)
   static constexpr int MIN_WAVES = AHEAD ? 1 : 3;
   struct Prm : R::Prm {
@@ -1713,6 +1713,9 @@ struct RatesStress : R {
     RetArgs ra;
     BlockStats* bs;  // one entry a workgroup
   };
+  __device__ static void pre(const Fields& f, const Prm& p, int i, Pre& in) {
+    stress_load<true, true, S32>(f, p.sp, i, in);
+  }
   typedef typename R::RT RT;
   template <int P>
   __device__ static void tail_put(const Fields& f, int i, bool act, const typename R::Acc& a,
@@ -1734,15 +1737,20 @@ struct RatesStress : R {
         RT v[9];
 #pragma unroll
         for (int k = 0; k < 9; k++) v[k] = sh[k * P];
-        if (p.sp.keep) R::put9(f, i, v);
 #pragma unroll
         for (int k = 0; k < 6; k++) d[k] = v[k];
 #pragma unroll
         for (int k = 0; k < 3; k++) w[k] = v[6 + k];
       };
       const bool active = (int)threadIdx.x < P && i < p.limit;
-      if (!AHEAD && active) pre(f, i, in);
+      if (!AHEAD && active) pre(f, p, i, in);
       stress_particle<true, true, REC, S32>(f, p.sp, p.ra, i, active, in, rates, st);
+      if (p.sp.keep && active) {
+        RT v[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) v[k] = sh[k * P];
+        R::put9(f, i, v);
+      }
     }
     stress_block_stats(st, NW, reinterpret_cast<BlockStats*>((RT*)lds + 9 * P), p.bs + b);
   }
@@ -1910,6 +1918,7 @@ struct CondG {
     double T_inf, h_conv, dt;
     int leap, first;
     float cs;
+    int skip;  // dT/dt and T_b are overwritten unread (StepParams::keep)
   };
   struct Own {
     float x, y, z, k, T, mdj;
@@ -1979,7 +1988,7 @@ struct CondG {
                                 const Prm& p) {
     if (!act) return;
     const double Ti = o.Ti, acc = cond_rate(f, i, a.val(), Ti, p, o.in);
-    f.dTdt[i] = acc;
+    if (!p.skip) f.dTdt[i] = acc;
     if (p.leap) {
       double Tn;
       if (p.first) {
@@ -1987,7 +1996,7 @@ struct CondG {
         Tn = Ti;
       } else {
         const double ta = o.in.ta;
-        f.Tb[i] = ta;
+        if (!p.skip) f.Tb[i] = ta;
         double tan = ta + acc * p.dt;
         f.Ta[i] = tan;
         Tn = (tan + ta) / 2.;
@@ -2463,10 +2472,10 @@ void launch_accel_integrate_mixed(hipStream_t s, const Fields& f, const TileList
                     IntegratePrm{dt, bc, fr, out, contacts}, fold);
 }
 void launch_cond_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
-                       double h_conv, double dt, bool leap, bool first, bool uh) {
+                       double h_conv, double dt, bool leap, bool first, bool uh, bool keep) {
   if (n <= 0) return;
   launch_gather<CondD>(s, f, tl, ntiles(n), uh, n, T_inf, h_conv, dt, leap ? 1 : 0,
-                       first ? 1 : 0);
+                       first ? 1 : 0, keep ? 0 : 1);
 }
 void launch_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n, int solid,
                        double dt, bool fuse, float cs32, bool uh) {
@@ -2544,20 +2553,21 @@ void launch_accel_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int
   accel_mixed<false>(s, f, tl, solid, alpha, beta, cs32, uh, uc, cs_uni, IntegratePrm{}, fold);
 }
 void launch_cond_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n, double T_inf,
-                       double h_conv, double dt, bool leap, bool first, float cs32, bool uh) {
+                       double h_conv, double dt, bool leap, bool first, float cs32, bool uh,
+                       bool keep) {
   if (n <= 0) return;
   launch_gather<CondG>(s, f, tl, ntiles(n), uh, n, T_inf, h_conv, dt, leap ? 1 : 0,
-                       first ? 1 : 0, cs32);
+                       first ? 1 : 0, cs32, keep ? 0 : 1);
 }
 void launch_cond_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl, int n,
                             int solid, double T_inf, double h_conv, double dt, bool leap,
                             bool first, bool uh, const unsigned long long* pz_d2,
-                            double pz_skin2) {
+                            double pz_skin2, bool keep, bool keep_next) {
   if (n <= 0) return;
   auto go = [&](auto tag, auto split) {
     typedef decltype(tag) K;
-    const typename K::Prm p{n, {n, T_inf, h_conv, dt, leap ? 1 : 0, first ? 1 : 0},
-                            {solid, n, dt, 1, 1}, pz_d2, pz_skin2};
+    const typename K::Prm p{n, {n, T_inf, h_conv, dt, leap ? 1 : 0, first ? 1 : 0, keep ? 0 : 1},
+                            {solid, n, dt, 1, 1, keep_next ? 0 : 1}, pz_d2, pz_skin2};
     launch_pair<K, split()>(s, ntiles(n), f, tl, p);
   };
   if (uh) go(CondDensD<true>{}, std::true_type{});
@@ -2566,12 +2576,13 @@ void launch_cond_dens_tiled(hipStream_t s, const Fields& f, const TileLists& tl,
 void launch_cond_dens_mixed(hipStream_t s, const Fields& f, const TileLists& tl, int n,
                             int solid, double T_inf, double h_conv, double dt, bool leap,
                             bool first, float cs32, bool uh, const unsigned long long* pz_d2,
-                            double pz_skin2) {
+                            double pz_skin2, bool keep, bool keep_next) {
   if (n <= 0) return;
   auto go = [&](auto tag, auto split) {
     typedef decltype(tag) K;
-    const typename K::Prm p{n, {n, T_inf, h_conv, dt, leap ? 1 : 0, first ? 1 : 0, cs32},
-                            {solid, n, dt, 1, cs32, 1}, pz_d2, pz_skin2};
+    const typename K::Prm p{
+        n, {n, T_inf, h_conv, dt, leap ? 1 : 0, first ? 1 : 0, cs32, keep ? 0 : 1},
+        {solid, n, dt, 1, cs32, 1, keep_next ? 0 : 1}, pz_d2, pz_skin2};
     launch_pair<K, split()>(s, ntiles(n), f, tl, p);
   };
   if (uh) go(CondDensG<true>{}, std::true_type{});

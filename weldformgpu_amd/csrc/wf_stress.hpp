@@ -96,18 +96,19 @@ struct StressIn {
   double strain[6], s[6];
 };
 template <bool FUSE_P, bool ENERGY, bool S32>
-__device__ __forceinline__ void stress_load(const Fields& f, int i, StressIn& in) {
+__device__ __forceinline__ void stress_load(const Fields& f, const StepParams& p, int i,
+                                            StressIn& in) {
   in.rho = f.rho[i];
-  in.cs = f.Cs[i];
-  in.p = FUSE_P ? f.rho0[i] : f.p[i];
-  in.G = f.G[i];
+  in.cs = p.uniform ? p.Cs : f.Cs[i];
+  in.p = !FUSE_P ? f.p[i] : p.uniform ? p.rho0 : f.rho0[i];
+  in.G = p.uniform ? p.G : f.G[i];
   in.T = f.T[i];
   in.sigma_y = f.sigma_y[i];
   in.ep = f.pl_strain[i];
 #pragma unroll
   for (int k = 0; k < 6; k++) in.strain[k] = f.strain[k][i];
   if (ENERGY) {
-    in.m = f.m[i];
+    in.m = p.uniform ? p.m : f.m[i];
     in.eint = f.eint[i];
   }
 #pragma unroll
@@ -176,7 +177,6 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
     for (int k = 0; k < 6; k++) f.strain[k][i] = in.strain[k] + d6[k] * dt;
     if (FUSE_P) {
       p_i = 0.0 + (cs_i * cs_i) * (rho_i - p_i);
-      if (p.keep) f.p[i] = p_i;
     }
     T9 WT = {W.xx, W.yx, W.zx, W.xy, W.yy, W.zy, W.xz, W.yz, W.zz};
     T9 SRT = tmul(S, WT, qp);
@@ -199,7 +199,6 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
     esr = sqrt(0.5 * ((D.xx - D.yy) * (D.xx - D.yy) + (D.yy - D.zz) * (D.yy - D.zz) +
                       (D.zz - D.xx) * (D.zz - D.xx)) +
                3.0 * (D.xy * D.xy + D.yz * D.yz + D.zx * D.zx));
-    if (p.keep) f.esr[i] = esr;
     const double J2 = 0.5 * (S.xx * S.xx + 2.0 * S.xy * S.yx + 2.0 * S.xz * S.zx +
                              S.yy * S.yy + 2.0 * S.yz * S.zy + S.zz * S.zz);
     sig_trial = sqrt(3.0 * J2);
@@ -298,18 +297,10 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
     }
     f.sigma_y[i] = sigy;
     f.pl_strain[i] = ep;
-    if (p.keep) f.sigma_eq[i] = sigeq;
     f.qpl[i] = p.taylor_quinney * sigeq * dep / dt;
     const double pi = p_i;
     // sigma = -p I + S (Mechanical.cu:540); store upper triangle
     const double sg[6] = {-pi + S.xx, -pi + S.yy, -pi + S.zz, S.xy, S.yz, S.xz};
-    if (p.keep) {
-#pragma unroll
-      for (int k = 0; k < 6; k++) {
-        if (S32) f.sigma32[k][i] = (float)sg[k];
-        else f.sigma[k][i] = sg[k];
-      }
-    }
     if (REC == kRec32) {  // sigma/rho^2, rho and Cs for the FP32 acceleration loop
       const double rho = rho_i, ir2 = 1.0 / (rho * rho);
       f.arec[rec32_at(i, 0)] = make_float4((float)(sg[0] * ir2), (float)(sg[1] * ir2),
@@ -327,6 +318,18 @@ __device__ __forceinline__ void stress_particle(const Fields& f, const StepParam
                   (S.xx * D.xx + S.yy * D.yy + S.zz * D.zz +
                    2.0 * (S.xy * D.xy + S.yz * D.yz + S.xz * D.xz));
       f.eint[i] = eint + de * dt;
+    }
+    // the conditional stores come last: a branch amid the arithmetic changes
+    // which products the compiler contracts
+    if (p.keep) {
+      if (FUSE_P) f.p[i] = p_i;
+      f.esr[i] = esr;
+      f.sigma_eq[i] = sigeq;
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        if (S32) f.sigma32[k][i] = (float)sg[k];
+        else f.sigma[k][i] = sg[k];
+      }
     }
     st.ep_bits = (unsigned long long)__double_as_longlong(ep > 0.0 ? ep : 0.0);
   }
