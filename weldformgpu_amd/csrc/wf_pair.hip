@@ -1,5 +1,7 @@
 // wf_pair.hip — the pair loops of the step (gfx950), FP64 and mixed
-// precision, on one kernel template (k_pair_gather).
+// precision, on two kernel templates: k_pair_lds, with everything a pair reads
+// of its neighbour staged in LDS (domains with one h), and k_pair_gather, which
+// gathers it (the others, described first).
 //
 // One workgroup per tile of kTileP Morton-consecutive particles, two threads
 // per particle.  The tile's staged set (the particles that are a neighbour of
