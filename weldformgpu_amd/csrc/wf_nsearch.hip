@@ -81,12 +81,19 @@ __global__ void k_ns_to_float(const double* __restrict__ x0, const double* __res
   }
 }
 
-__global__ __launch_bounds__(256) void k_ns_minmax_part(const float* p0, const float* p1,
-                                                        const float* p2, int n, float* part) {
+// the positions in FP32, and their bounding box by block
+__global__ __launch_bounds__(256) void k_ns_minmax_part(const double* __restrict__ x0,
+                                                        const double* __restrict__ x1,
+                                                        const double* __restrict__ x2, float* p0,
+                                                        float* p1, float* p2, int n,
+                                                        float* part) {
   __shared__ float sh[6][256];
   float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    float v[3] = {p0[i], p1[i], p2[i]};
+    const float v[3] = {(float)x0[i], (float)x1[i], (float)x2[i]};
+    p0[i] = v[0];
+    p1[i] = v[1];
+    p2[i] = v[2];
     for (int c = 0; c < 3; c++) {
       mn[c] = fminf(mn[c], v[c]);
       mx[c] = fmaxf(mx[c], v[c]);
@@ -183,14 +190,30 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int* in, int64
   }
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
-__global__ void k_scan_parts(int* part, int nb) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    int run = 0;
-    for (int b = 0; b < nb; b++) {
-      int t = part[b];
-      part[b] = run;
-      run += t;
+// the exclusive scan of the nb block sums, in place, by one block (one thread
+// walking them took 18 us for the 742 sums of 759k particles)
+__global__ __launch_bounds__(kScanBlock) void k_scan_parts(int* part, int nb) {
+  __shared__ int ws[kScanBlock / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int carry = 0;
+  for (int b0 = 0; b0 < nb; b0 += kScanBlock) {
+    const int b = b0 + threadIdx.x;
+    const int v = b < nb ? part[b] : 0;
+    int incl = v;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(incl, d);
+      if (lane >= d) incl += o;
     }
+    if (lane == 63) ws[w] = incl;
+    __syncthreads();
+    int off = carry;
+    for (int u = 0; u < kScanBlock / 64; u++) {
+      const int t = ws[u];
+      off += u < w ? t : 0;
+      carry += t;
+    }
+    if (b < nb) part[b] = off + incl - v;
+    __syncthreads();  // ws may be written again
   }
 }
 __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const int* in, int64_t m,
@@ -235,9 +258,22 @@ __global__ void k_ns_order(const int* key, const int* cell_start, const int* per
   gather[b + r] = i;
 }
 
-__global__ void k_ns_gather_f32(float* dst, const float* src, const int* idx, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[idx[i]];
+// the FP32 positions in the new order; clears two counters (may be null)
+__global__ void k_ns_gather_f32(float* d0, float* d1, float* d2, const float* __restrict__ s0,
+                                const float* __restrict__ s1, const float* __restrict__ s2,
+                                const int* __restrict__ idx, int n, int* zero0, int* zero1) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) {
+    const int j = idx[i];
+    const float a = s0[j], b = s1[j], c = s2[j];
+    d0[i] = a;
+    d1[i] = b;
+    d2[i] = c;
+  }
+  if (i == 0) {
+    if (zero0) *zero0 = 0;
+    if (zero1) *zero1 = 0;
+  }
 }
 
 // *out = sum of v[0..n) (one block, a fixed order: deterministic)
@@ -309,7 +345,7 @@ void launch_scan_exclusive(hipStream_t s, const int* in, int64_t m, int* part, i
   const int nb = grid1(m, kScanBlock);
   if (nb <= 0) return;
   hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kScanBlock), 0, s, in, m, part);
-  hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(64), 0, s, part, nb);
+  hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kScanBlock), 0, s, part, nb);
   hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, s, in, m, part, out);
 }
 
@@ -443,11 +479,9 @@ int ns_build(hipStream_t s, NsWork** work, const double* const pos_src[3], int n
   if (rc) return rc;
   const float rf = (float)radius;
   const float r2 = rf * rf;
-  hipLaunchKernelGGL(k_ns_to_float, dim3(grid1(n, 256)), dim3(256), 0, s, pos_src[0], pos_src[1],
-                     pos_src[2], w->pf[0], w->pf[1], w->pf[2], n);
   int nbm = std::min(kMmBlocks, std::max(1, grid1(n, 256)));
-  hipLaunchKernelGGL(k_ns_minmax_part, dim3(nbm), dim3(256), 0, s, w->pf[0], w->pf[1], w->pf[2],
-                     n, w->mm_part);
+  hipLaunchKernelGGL(k_ns_minmax_part, dim3(nbm), dim3(256), 0, s, pos_src[0], pos_src[1],
+                     pos_src[2], w->pf[0], w->pf[1], w->pf[2], n, w->mm_part);
   hipLaunchKernelGGL(k_ns_minmax_final, dim3(1), dim3(256), 0, s, w->mm_part, nbm, w->mm);
   if (hipMemcpyAsync(w->mm_host, w->mm, 6 * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess)
     return WF_E_HIP;
@@ -478,7 +512,7 @@ int ns_build(hipStream_t s, NsWork** work, const double* const pos_src[3], int n
   int nsb = grid1(nkeys, kScanBlock);
   hipLaunchKernelGGL(k_scan_reduce, dim3(nsb), dim3(kScanBlock), 0, s, w->cell_count, nkeys,
                      w->scan_part);
-  hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(64), 0, s, w->scan_part, nsb);
+  hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kScanBlock), 0, s, w->scan_part, nsb);
   hipLaunchKernelGGL(k_scan_apply, dim3(nsb), dim3(kScanBlock), 0, s, w->cell_count, nkeys,
                      w->scan_part, w->cell_start);
   hipLaunchKernelGGL(k_ns_place, dim3(grid1(n, 256)), dim3(256), 0, s, w->key, w->rank,
@@ -486,11 +520,9 @@ int ns_build(hipStream_t s, NsWork** work, const double* const pos_src[3], int n
   // new permutation and gather map
   hipLaunchKernelGGL(k_ns_order, dim3(grid1(n, 256)), dim3(256), 0, s, w->key, w->cell_start,
                      perm, w->slot_orig, n, perm_tmp, gather);
-  for (int c = 0; c < 3; c++)
-    hipLaunchKernelGGL(k_ns_gather_f32, dim3(grid1(n, 256)), dim3(256), 0, s, w->pfn[c], w->pf[c],
-                       gather, n);
-  hipLaunchKernelGGL(k_ns_fill_i32, dim3(1), dim3(64), 0, s, &ctr->nb_over_cap, 0, (int64_t)1);
-  hipLaunchKernelGGL(k_ns_fill_i32, dim3(1), dim3(64), 0, s, w->tile_ovf, 0, (int64_t)1);
+  hipLaunchKernelGGL(k_ns_gather_f32, dim3(grid1(n, 256)), dim3(256), 0, s, w->pfn[0], w->pfn[1],
+                     w->pfn[2], w->pf[0], w->pf[1], w->pf[2], gather, n, &ctr->nb_over_cap,
+                     w->tile_ovf);
   // tiles of the new order: occupied neighbour cells and staged counts
   const int nt = (n + kTileP - 1) / kTileP;
   const float* pfn[3] = {w->pfn[0], w->pfn[1], w->pfn[2]};
@@ -499,7 +531,7 @@ int ns_build(hipStream_t s, NsWork** work, const double* const pos_src[3], int n
   int ntb = grid1(nt, kScanBlock);
   hipLaunchKernelGGL(k_scan_reduce, dim3(ntb), dim3(kScanBlock), 0, s, w->tile_ucnt,
                      (int64_t)nt, w->tile_scan);
-  hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(64), 0, s, w->tile_scan, ntb);
+  hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kScanBlock), 0, s, w->tile_scan, ntb);
   hipLaunchKernelGGL(k_scan_apply, dim3(ntb), dim3(kScanBlock), 0, s, w->tile_ucnt, (int64_t)nt,
                      w->tile_scan, w->tile_uoff);
   if (hipMemcpyAsync(w->tile_host, w->tile_uoff + nt, sizeof(int), hipMemcpyDeviceToHost, s) !=
@@ -558,9 +590,9 @@ int ns_relist_local(hipStream_t s, NsWork* w, const double* const x[3], const do
                      w->cell_start, perm, n, w->slot_orig);
   hipLaunchKernelGGL(k_ns_order, dim3(grid1(n, 256)), dim3(256), 0, s, w->key, w->cell_start,
                      perm, w->slot_orig, n, w->lperm, w->lgather);
-  for (int c = 0; c < 3; c++)
-    hipLaunchKernelGGL(k_ns_gather_f32, dim3(grid1(n, 256)), dim3(256), 0, s, w->pfn[c], w->pf[c],
-                       w->lgather, n);
+  hipLaunchKernelGGL(k_ns_gather_f32, dim3(grid1(n, 256)), dim3(256), 0, s, w->pfn[0], w->pfn[1],
+                     w->pfn[2], w->pf[0], w->pf[1], w->pf[2], w->lgather, n, (int*)nullptr,
+                     (int*)nullptr);
   // the tiles within reach of the plastic zone
   hipLaunchKernelGGL(k_hot_cells, dim3(grid1(n, 256)), dim3(256), 0, s, w->pf[0], w->pf[1],
                      w->pf[2], n, g, pl_strain, ep_hot, w->cell_flag);
