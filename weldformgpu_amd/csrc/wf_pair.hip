@@ -1437,8 +1437,10 @@ void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
           PT x, y, z;
           typename K::Nb nb;
           if constexpr (DropOf<K>::on) {
-            // entries past the list add exact zeros (drop)
-            fetch(u < nk ? sl_of(w0, u) : 0, x, y, z, nb);
+            // entries past the list repeat one of it (TileLists) and add exact
+            // zeros (drop): another particle's value, were it not finite, would
+            // reach a particle that does not list it as 0 x NaN
+            fetch(sl_of(w0, u), x, y, z, nb);
             if (u >= nk) K::drop(nb);
             K::pair(x, y, z, nb, own, sum, prm);
           } else if (u < nk) {

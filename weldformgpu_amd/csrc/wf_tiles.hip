@@ -465,7 +465,7 @@ __global__ __launch_bounds__(kListThreads) void k_tile_lists(
     unsigned v[4] = {w.x & 0xFFFFu, w.x >> 16, w.y & 0xFFFFu, w.y >> 16};
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      if (4 * q + u >= m) v[u] = 0u;
+      if (4 * q + u >= m) v[u] = v[0];  // the quad's first, which is in the list
       else if (compact) v[u] = (unsigned short)sidx[v[u]];
     }
     qrow[(int64_t)q * npad] = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);

@@ -56,7 +56,8 @@ __device__ __forceinline__ void cell_of(const GridDesc& g, float px, float py, f
 
 // What the pair kernels read.  slotq holds four 16-bit staged-set positions
 // per 8 bytes: entry k of particle i is 16-bit lane (k&3) of
-// slotq[(k>>2)*npad + i]; rows are in ascending staged (= particle) order.
+// slotq[(k>>2)*npad + i]; rows are in ascending staged (= particle) order, and
+// the rest of a list's last quad repeats that quad's first entry.
 struct TileLists {
   const int* count;
   const uint2* slotq;
