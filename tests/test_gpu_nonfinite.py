@@ -117,3 +117,18 @@ def test_passes_with_one_h(wflib, n, precision):
 @pytest.mark.parametrize("n", [60, 3000, 6000, 12000, 19000])
 def test_steps_with_one_h(wflib, n, precision):
     _check_steps(wflib, n, precision, {})
+
+
+# the loops that gather: one particle's h, sound speed or mass apart
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("apart", ["h", "Cs", "m"])
+@pytest.mark.parametrize("n", [60, 6000, 19000])
+def test_passes_of_general_domains(wflib, n, apart, precision):
+    _check_passes(wflib, n, precision, {apart: 1.0 + 1e-6})
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("apart", ["h", "Cs", "m"])
+@pytest.mark.parametrize("n", [60, 6000, 19000])
+def test_steps_of_general_domains(wflib, n, apart, precision):
+    _check_steps(wflib, n, precision, {apart: 1.0 + 1e-6})

@@ -1124,7 +1124,7 @@ void k_pair_gather(Fields f, TileLists tl, typename K::Prm prm) {
     uint2 w1 = word(k0 + KS);
     int jn[4];
 #pragma unroll
-    for (int u = 0; u < 4; u++) jn[u] = k0 + u < cnt ? st[sl_of(w0, u)].j : 0;
+    for (int u = 0; u < 4; u++) jn[u] = k0 < cnt ? st[sl_of(w0, u)].j : 0;
     for (int k = k0; k < kend; k += KS) {
       const int nk = min(4, cnt - k);
       int jc[4];
@@ -1137,9 +1137,9 @@ void k_pair_gather(Fields f, TileLists tl, typename K::Prm prm) {
 #pragma unroll
       for (int u0 = 0; u0 < 4; u0 += NB) {
         // with straight-line batches (drop()) every record of the batch is
-        // loaded, also for entries past the list: their index is the
-        // particle index an earlier entry held (or particle 0), so the load
-        // stays in bounds, and each pair waits only for its own record;
+        // loaded, also for entries past the list: they repeat one of it
+        // (TileLists, or the index an earlier entry held), and each pair waits
+        // only for its own record;
         // otherwise only the list's entries are loaded (the FP64
         // acceleration loop is bound by its gathers)
         typename K::Nb nb[NB];
@@ -1149,12 +1149,12 @@ void k_pair_gather(Fields f, TileLists tl, typename K::Prm prm) {
           else if (DropOf<K>::on || u0 + u == 0 || u0 + u < nk) K::load(f, jc[u0 + u], nb[u]);
         }
         // the batch's staged positions are read before any pair is evaluated
-        // (entries past the list read slot 0 and are not evaluated)
+        // (entries past the list repeat one of it)
         typename K::PT px[NB], py[NB], pz[NB];
         int sl[NB];
 #pragma unroll
         for (int u = 0; u < NB; u++) {
-          sl[u] = u0 + u < nk ? sl_of(w0, u0 + u) : 0;
+          sl[u] = sl_of(w0, u0 + u);
           const Slot& sv = st[sl[u]];
           px[u] = sv.x;
           py[u] = sv.y;
