@@ -161,3 +161,43 @@ def test_constants_that_differ(oracle, wflib, field, precision):
         for k in MECH_FIELDS:
             if np.linalg.norm(st[k]) > 0.0:
                 assert rel_l2(d.get(k), st[k]) <= TOL[precision], k
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+def test_call_that_a_candidate_search_ends(wflib, precision):
+    """The rigid mesh, far from the particles, turns non-finite in mid-call, and
+    the candidate search of the sixth step refuses it (the lists, rebuilt from
+    an unchanged snapshot, end no call).  The fields are those that single-step
+    calls leave, which have the step's passes up to the acceleration, and the
+    Newton statistics count the step."""
+    def case(omega):
+        sc = scenarios.c4_contact(scale=0.2, r=0.25e-3, dens=16, offset=0.137)
+        sc.cfg.precision = precision
+        randomize(sc, seed=4, v_scale=0.5)
+        sc.fields["T"] = 300.0 + np.random.default_rng(4).uniform(0.0, 50.0, sc.n)
+        sc.meshes[0]["nodes"][:, 2] += 1.0
+        sc.meshes[0]["vel"] = (0.0, 0.0, 0.0)
+        # the nodes' distance grows by a factor of omega dt a step
+        sc.meshes[0]["omega"] = (0.0, 0.0, omega / sc.cfg.dt)
+        return sc
+    fields = FIELDS + ["Ta", "Tb", "dTdt", "contforce", "normal"]
+    runs, newton = [], []
+    for calls in ([20], [1] * 6):
+        with to_gpu(case(1e65), wflib) as d:
+            for k in calls[:-1]:
+                d.step(k)
+            with pytest.raises(WfError, match="non-finite rigid mesh"):
+                d.step(calls[-1])
+            assert d.stats()["step"] == 5
+            newton.append(d.stats()["newton_calls"])
+            runs.append({k: d.get(k) for k in fields})
+    for k in fields:
+        assert np.array_equal(runs[0][k], runs[1][k]), k
+    with to_gpu(case(0.0), wflib) as d:
+        d.step(5)
+        before = d.get("a")
+        d.step(1)
+        assert newton == [d.stats()["newton_calls"]] * 2 and newton[0] > 0
+        for k in ("sigma", "strrate", "rho", "pl_strain"):
+            assert np.array_equal(runs[0][k], d.get(k)), k
+    assert not np.array_equal(runs[0]["a"], before)  # of the step the search ended

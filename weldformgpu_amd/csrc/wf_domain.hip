@@ -1794,12 +1794,14 @@ static bool yield_asked(const wf_domain* d, bool last) {
 // Whether a step's stress pass stores the fields that only a caller reads
 // (StepParams::keep): in a call's last step, and where the call could end
 // early, at a list rebuild or a contact candidate search that refuses its
-// input.  In the others the next step overwrites them unread.
-// ts_i: the step's count since the last due rebuild.
+// input: the step that searches (which ends before its conduction pass) and
+// the one before a search or rebuild.  In the others the next step overwrites
+// them unread.  ts_i: the step's count since the last due rebuild.
 static bool step_keeps(const wf_domain* d, bool last, int ts_i) {
   if (last || d->plastic_zone()) return true;
   if (d->cfg.contact && ts_i == 0) return true;
   if (ts_i + 1 <= d->cfg.ns_interval - 1) return false;
+  if (d->cfg.contact) return true;
   const bool stale = (d->cfg.quirks & WF_Q_STALE_NS_POS) != 0;
   return !(stale && d->nb_built && d->built_gen == d->snap_gen);  // a no-op rebuild
 }
@@ -1878,16 +1880,19 @@ int wf_step(wf_domain* d, int n_steps) {
       // The contact step's surface pass and candidates read nothing that the
       // acceleration pass writes, so they run before it (SolverFraser.cu:
       // 233-257 has them behind it): that pass can then leave the particles
-      // with candidates to the contact pass.
+      // with candidates to the contact pass.  A search that refuses its input
+      // ends the call behind the acceleration pass, not integrated, so that
+      // what the caller finds is of one step, its statistics among it.
       const bool contact = d->cfg.contact && d->n_meshes > 0;
+      int refused = WF_OK;
       if (d->cfg.contact) {
         timer_begin(d);
         if (!fuse_surf) {
           if ((rc = d->surface_init())) return rc;
           d->launch_surface();
         }
-        if (contact && d->ts_i == 0 && (rc = d->contact_nb())) return rc;
-        if (contact && (rc = d->contact_list())) return rc;
+        if (contact && d->ts_i == 0) refused = d->contact_nb();
+        if (contact && !refused && (rc = d->contact_list())) return rc;
         if ((rc = timer_end(d, WF_K_CONTACT))) return rc;
       }
       // Without the axisymmetric clamp between them, the acceleration pass
@@ -1898,8 +1903,8 @@ int wf_step(wf_domain* d, int n_steps) {
       // after the passes.  Not the FP64 pass that gathers its neighbours'
       // records: its lower occupancy made it slower (0.396 against 0.332 +
       // 0.032 ms on a 759k-particle cylinder).
-      const bool fuse_int = d->cfg.fuse_integrate && !d->cfg.axisymm && d->solid == d->n &&
-                            (mx || d->f.arec64u);
+      const bool fuse_int = !refused && d->cfg.fuse_integrate && !d->cfg.axisymm &&
+                            d->solid == d->n && (mx || d->f.arec64u);
       const int* contacts = contact ? d->cl.count : nullptr;
       IntegrateOut out{};
       timer_begin(d, true);
@@ -1929,6 +1934,7 @@ int wf_step(wf_domain* d, int n_steps) {
         if (d->cfg.axisymm) launch_axisymm_bc(d->stream, d->f, d->n);  // SolverFraser.cu:229-231
         if ((rc = timer_end(d, WF_K_ACCEL))) return rc;
       }
+      if (refused) return refused;
       if (contact) {
         timer_begin(d);
         if (fuse_int)
