@@ -201,3 +201,34 @@ def test_call_that_a_candidate_search_ends(wflib, precision):
         for k in ("sigma", "strrate", "rho", "pl_strain"):
             assert np.array_equal(runs[0][k], d.get(k)), k
     assert not np.array_equal(runs[0]["a"], before)  # of the step the search ended
+
+
+@pytest.mark.parametrize("n", [3000, 9000, 17000])
+def test_mixed_contact_integration_in_the_acceleration_pass(wflib, n):
+    """Mixed precision: contact steps that integrate in the acceleration pass
+    (the particles with contact candidates in the contact pass) against the
+    separate pass, over steps with rebuilds: bit-identical, the positions that
+    are updated in place and what the next steps read of the spare mirrors
+    included."""
+    runs = []
+    for fuse in (1, 0):
+        scale = (n / 1320424) ** (1 / 3)
+        sc = scenarios.c4_contact(scale=scale, dens=max(6, int(64 * scale)), offset=0.137)
+        randomize(sc, seed=n, v_scale=0.5)
+        sc.cfg.precision = _abi.WF_MIXED
+        sc.cfg.fuse_integrate = fuse
+        sc.cfg.quirks &= ~_abi.WF_Q_STALE_NS_POS
+        sc.cfg.ns_min_plastic = 0.0
+        sc.fields["pl_strain"] = np.full(sc.n, 1e-3)
+        with to_gpu(sc, wflib) as d:
+            d.set_timing(True)
+            for k in (1, 7, 3):
+                d.step(k)
+            runs.append({k: d.get(k) for k in FIELDS + ["contforce", "q_friction"]})
+            assert d.kernel_time("accel_integrate")[1] == (11 if fuse else 0)
+            assert d.kernel_time("integrate")[1] == (0 if fuse else 11)
+            assert d.stats()["ns_builds"] >= 2
+            assert (d.get("cont_nb_count") > 0).sum() > 0
+            assert np.abs(runs[-1]["contforce"]).sum() > 0
+    for k in runs[0]:
+        assert np.array_equal(runs[0][k], runs[1][k]), k
