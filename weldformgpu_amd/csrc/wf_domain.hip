@@ -919,12 +919,22 @@ int wf_create(const wf_config* cfg, wf_domain** out) {
     }
   }
   if (!rc && sizeof(double) * 6 * (size_t)d->n >= wf_domain::kBigCopy) {
-    if (hipHostMalloc(&d->bounce, 2 * wf_domain::kCopyThreads * wf_domain::kCopyChunk) !=
-        hipSuccess)
-      rc = WF_E_NOMEM;
-    for (hipEvent_t& e : d->bounce_ev)
-      if (!rc && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) rc = WF_E_HIP;
-    if (!rc && hipGetDevice(&d->device) != hipSuccess) rc = WF_E_HIP;
+    // a host without this much memory to lock reads back by the runtime's copy
+    constexpr size_t kBytes = 2 * wf_domain::kCopyThreads * wf_domain::kCopyChunk;
+    void* q = nullptr;
+    bool ok = hipGetDevice(&d->device) == hipSuccess && hipHostMalloc(&q, kBytes) == hipSuccess;
+    for (hipEvent_t& e : d->bounce_ev) {
+      if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        e = nullptr;
+        ok = false;
+      }
+    }
+    if (ok) {
+      d->bounce = (char*)q;
+    } else {
+      if (q) hipHostFree(q);
+      (void)hipGetLastError();  // a later launch's check must not find it
+    }
   }
   if (!rc) {
     void* q = nullptr;
