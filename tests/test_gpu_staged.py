@@ -140,3 +140,17 @@ def test_contact_pass_over_the_listed_particles(oracle, wflib, precision, policy
         assert rel_l2(cf, st.contact_arrays["cf"]) <= tol
         for k in ("u", "v", "sigma"):
             assert rel_l2(d.get(k), st[k]) <= tol, k
+
+
+@pytest.mark.parametrize("uniform_mass", [True, False])
+def test_contact_timing_counts_what_was_launched(wflib, uniform_mass):
+    """The contact timer's intervals: forces and mesh motion in every step, the
+    candidate search in every fifth, and the free-surface pass where the rates
+    pass does not take its sums along (in the search's interval)."""
+    sc = scenarios.c4_contact(scale=0.2, r=0.25e-3, dens=16, offset=0.137)
+    if not uniform_mass:
+        sc.fields["m"][sc.n // 3] *= 1.0 + 1e-9
+    with to_gpu(sc, wflib) as d:
+        d.set_timing(True)
+        d.step(10)
+        assert d.kernel_time("contact")[1] == (2 * 10 + 2 if uniform_mass else 3 * 10)

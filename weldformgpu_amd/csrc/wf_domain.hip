@@ -1895,14 +1895,16 @@ int wf_step(wf_domain* d, int n_steps) {
       // what the caller finds is of one step, its statistics among it.
       const bool contact = d->cfg.contact && d->n_meshes > 0;
       int refused = WF_OK;
-      if (d->cfg.contact) {
+      const bool search = contact && d->ts_i == 0;
+      const bool relist = contact && (search || !d->act_valid || d->cf_set);
+      if (d->cfg.contact && (!fuse_surf || relist)) {  // else there is nothing to time
         timer_begin(d);
         if (!fuse_surf) {
           if ((rc = d->surface_init())) return rc;
           d->launch_surface();
         }
-        if (contact && d->ts_i == 0) refused = d->contact_nb();
-        if (contact && !refused && (rc = d->contact_list())) return rc;
+        if (search) refused = d->contact_nb();
+        if (relist && !refused && (rc = d->contact_list())) return rc;
         if ((rc = timer_end(d, WF_K_CONTACT))) return rc;
       }
       // Without the axisymmetric clamp between them, the acceleration pass
