@@ -38,6 +38,19 @@ def _scenario(n, precision, beta):
     return sc
 
 
+def _large(n, precision):
+    sc = scenarios.c3_johnson_cook(scale=0.46)
+    for k, v in sc.fields.items():
+        sc.fields[k] = v[:n].copy()
+    sc.cfg.n_particles = sc.cfg.solid_count = n
+    sc.cfg.precision = precision
+    randomize(sc, seed=n)
+    rng = np.random.default_rng(n)
+    sc.fields["T"] = 300.0 + rng.uniform(0.0, 50.0, n)
+    sc.fields["k_T"] = rng.choice([150.0, 200.0], n)
+    return sc
+
+
 def _passes(d, st, cfg, tol):
     d.CalcDensInc()
     st.calc_dens_inc(cfg)
@@ -154,3 +167,26 @@ def test_contact_timing_counts_what_was_launched(wflib, uniform_mass):
         d.set_timing(True)
         d.step(10)
         assert d.kernel_time("contact")[1] == (2 * 10 + 2 if uniform_mass else 3 * 10)
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("n", [17000, 65536, 65537])
+@pytest.mark.parametrize("compact_max", [1, 0])
+def test_large_sets_of_whole_tiles(oracle, wflib, n, compact_max, precision):
+    """Two lanes a particle, up to 512 tiles (65,536 particles) with 1,024 and
+    beyond with 960 staged entries: sets left uncompacted (~1,230 particles),
+    and, off the lattice under a list skin, sets on both sides of the two."""
+    sc = _large(n, precision)
+    if compact_max:
+        sc.cfg.ns_compact_max = compact_max
+    else:
+        dx = sc.meta["dx"]
+        sc.cfg.rebuild_policy = _abi.WF_REBUILD_PLASTIC_ZONE
+        sc.cfg.ns_skin, sc.cfg.ep_hot = 0.3 * dx, 1e9
+        sc.fields["x"] += np.random.default_rng(n).uniform(-0.2 * dx, 0.2 * dx, (n, 3))
+    st = to_oracle(oracle, sc)
+    st.nsearch(sc.cfg)
+    with to_gpu(sc, wflib) as d:
+        d.nsearch()
+        assert d.nsearch_stats()[1] == 0
+        _passes(d, st, sc.cfg, TOL[precision])

@@ -248,7 +248,8 @@ constexpr int kStage64 = WF_STAGE64;
 // next lattice shell ~760 (at most ~990, 1 % of the tiles above 960).  1,024
 // leave the workgroups a CU that 960 leave, but for the loops with 56 bytes
 // (FP64 density and rates: two instead of three) and 32 (FP32 density, rates
-// and conduction: four instead of five; rates 0.061 against 0.057 ms).
+// and conduction: four instead of five; rates 0.061 against 0.057 ms): those
+// take 960 where there are more tiles than two a CU (launch_pair).
 #define WF_LDS64(nv, nw) \
   typedef double2 LV;    \
   typedef double LW;     \
@@ -1313,10 +1314,10 @@ struct TailOf<K, std::void_t<decltype(K::TAIL)>> {
   static constexpr bool on = true, pre = K::PRE;
   typedef typename K::Pre type;
 };
-template <class K, int L, int P>
+template <class K, int L, int P, int ST>
 __global__ __launch_bounds__(L * P) __attribute__((amdgpu_waves_per_eu(WavesOf<K>::value)))
 void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
-  constexpr int S = kTileP / P, NT = L * P, ST = K::SET;
+  constexpr int S = kTileP / P, NT = L * P;
   static_assert(L >= 2 && L <= 16 && (L & (L - 1)) == 0, "a power of two of lanes per particle");
   typedef typename K::LV LV;
   typedef typename K::LW LW;
@@ -1454,32 +1455,48 @@ void k_pair_lds(Fields f, TileLists tl, typename K::Prm prm) {
       w1 = w2;
     }
   } else {
-    // a larger set in passes; each lane takes the list entries of its quads
-    // that fall in the pass
-    SlotReader sr;
-    sr.init(tl, i, cnt);
-    for (int c0 = 0; c0 < ucnt; c0 += ST) {
-      const int m = min(ST, ucnt - c0);
-      __syncthreads();
-      stage(c0, m);
-      __syncthreads();
-      const int lim = c0 + m;
-      while (sr.k < sr.cnt) {
-        if (((sr.k >> 2) & (L - 1)) != sub) {
-          sr.skip_quad();
-          continue;
-        }
-        const int sl = sr.slot();
-        if (sl >= lim) break;
-        sr.advance();
+    // A larger set: its first ST entries are staged, what a pair reads of one
+    // beyond comes from memory.  Rows ascend, so that is the end of some lists.
+    // Staging the set in passes instead made such a tile take more than twice
+    // as long, which showed in every domain of a few rounds of workgroups: mixed
+    // step with a 0.4 dx skin at 61,748 particles 80.9 -> 63.0 us, with the
+    // positions off the lattice at 20,400 77.6 -> 49.9, sets left uncompacted
+    // (~1,230 particles) at 801,536 629 -> 500 us (gathering: 70.3, 58.0, 732);
+    // FP64 92.9 -> 82.4, 77.0 -> 62.7, 1,156 -> 885 (101, 80.4, 1,281).
+    stage(0, ST);
+    __syncthreads();
+    const uint2* __restrict__ q = tl.slotq + min((int64_t)i, tl.npad - 1);
+    const int klast = max(cnt - 1, 0);
+    const unsigned np = (unsigned)tl.npad;
+    auto word = [&](int k) { return q[(unsigned)(min(k, klast) >> 2) * np]; };
+    constexpr int KS = 4 * L;
+    uint2 w0 = word(4 * sub);
+    for (int k = 4 * sub; k < cnt; k += KS) {
+      const uint2 w1 = word(k + KS);
+      const int nk = min(4, cnt - k);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if (u >= nk) break;
+        const unsigned h = (u & 2) ? w0.y : w0.x;
+        const int sl = (int)((u & 1) ? h >> 16 : h & 0xFFFFu);
         quad([&](auto& sum) {
           PT x, y, z;
           typename K::Nb nb;
-          fetch(sl - c0, x, y, z, nb);
-          if constexpr (R) K::rest_get(gat<Rest>(K::rest(f), sj[sl - c0]), nb);
+          if (sl < ST) {
+            fetch(sl, x, y, z, nb);
+            if constexpr (R) K::rest_get(gat<Rest>(K::rest(f), sj[sl]), nb);
+          } else {
+            const int j = tj[sl];
+            LV e[NV];
+            LW r[1] = {};
+            K::lds_put(f, j, cx, e, r);
+            K::lds_get(e, r, x, y, z, nb);
+            if constexpr (R) K::rest_get(gat<Rest>(K::rest(f), j), nb);
+          }
           K::pair(x, y, z, nb, own, sum, prm);
         });
       }
+      w0 = w1;
     }
   }
   merge_lanes<K, L>(acc);
@@ -2340,10 +2357,13 @@ static void launch_timed(void (*kernel)(Fields, TileLists, typename K::Prm), dim
 // 26.3; 41 tiles 45.1 / 38.6 / 35.7 / 37.5; 35.3 / 31.2 / 29.2 / 30.0; 65
 // tiles 45.4 / 38.7 / 40.3 / 45.2; 34.9 / 30.8 / 31.4 / 31.8; 142 tiles 46.9 /
 // 48.1 / 51.5 / 60.7; 35.6 / 35.4 / 35.4 / 42.7.
+constexpr int kCus = 256;
 static int pair_split(int nt) {
-  constexpr int kCus = 256;
   return 8 * nt <= kCus ? 8 : 4 * nt <= kCus ? 4 : 2 * nt <= kCus ? 2 : 1;
 }
+// Up to two tiles a CU, 1,024 staged entries cost no loop a workgroup a CU (an
+// entry has at most 76 bytes) and send fewer tiles to memory.
+constexpr int kSetMax = 1024;
 template <class K, bool LDS = true>
 static void launch_pair(hipStream_t s, int nt, const Fields& f, const TileLists& tl,
                         const typename K::Prm& p) {
@@ -2353,10 +2373,11 @@ static void launch_pair(hipStream_t s, int nt, const Fields& f, const TileLists&
     auto go = [&](auto kernel) {
       launch_timed<K>(kernel, dim3(nt * split), dim3(kThreads), s, f, tl, p);
     };
-    if (split == 8) go(k_pair_lds<K, 16, kTileP / 8>);
-    else if (split == 4) go(k_pair_lds<K, 8, kTileP / 4>);
-    else if (split == 2) go(k_pair_lds<K, 4, kTileP / 2>);
-    else go(k_pair_lds<K, 2, kTileP>);
+    if (split == 8) go(k_pair_lds<K, 16, kTileP / 8, kSetMax>);
+    else if (split == 4) go(k_pair_lds<K, 8, kTileP / 4, kSetMax>);
+    else if (split == 2) go(k_pair_lds<K, 4, kTileP / 2, kSetMax>);
+    else if (nt <= 2 * kCus) go(k_pair_lds<K, 2, kTileP, kSetMax>);
+    else go(k_pair_lds<K, 2, kTileP, K::SET>);
   } else {
     launch_timed<K>(k_pair_gather<K>, dim3(nt), dim3(kTileP * K::LANES), s, f, tl, p);
   }
