@@ -1,8 +1,9 @@
 """The pinned chunks of a large domain's read-back are a help, not a need.
 
 The library runs in a child process over a stand-in for the HIP runtime whose
-device memory is host memory and whose kernels do nothing, so that a pinned
-allocation, an event or a device switch can be refused at will.  A field set
+device memory is host memory and whose kernels do nothing, but for the one that
+copies a chunk, so that a pinned allocation, an event or a device switch can be
+refused at will.  A field set
 and read back then goes through the staging buffer and back: the bytes that
 come out are those that went in, whichever way they were copied.
 """
@@ -31,14 +32,30 @@ extern "C" {
 int wf_test_live() { return live; }
 int wf_test_pinned_copies() { return pinned_copies; }
 void** __hipRegisterFatBinary(const void*) { static void* h; return &h; }
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*,
-                           void*, int*) {}
+static const void* copy_chunk = nullptr;
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*,
+                           void*, void*, int*) {
+  if (strstr(name, "k_copy_chunk")) copy_chunk = f;
+}
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void**) {}
 struct Dim3 { unsigned x, y, z; };
-int __hipPushCallConfiguration(Dim3, Dim3, size_t, void*) { return 0; }
-int __hipPopCallConfiguration(Dim3*, Dim3*, size_t*, void**) { return 0; }
-int hipLaunchKernel(const void*, Dim3, Dim3, void**, size_t, void*) { return 0; }
+static thread_local Dim3 grid_, block_;
+int __hipPushCallConfiguration(Dim3 g, Dim3 b, size_t, void*) { grid_ = g; block_ = b; return 0; }
+int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* lds, void** s) {
+  *g = grid_; *b = block_; *lds = 0; *s = nullptr;
+  return 0;
+}
+int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t, void*) {
+  if (f != copy_chunk) return 0;
+  const char* src = *(const char**)args[0];
+  char* dst = *(char**)args[1];
+  const int bytes = *(int*)args[2];
+  if (dst < pin_lo || dst + bytes > pin_hi || 16ull * grid.x * block.x < (unsigned)bytes) abort();
+  pinned_copies++;
+  memcpy(dst, src, bytes);
+  return 0;
+}
 int hipExtLaunchKernel(const void*, Dim3, Dim3, void**, size_t, void*, void*, void*, int) { return 0; }
 int hipGetDeviceCount(int* n) { *n = 1; return 0; }
 int hipGetDevice(int* d) { *d = 0; return 0; }
@@ -60,7 +77,6 @@ int hipHostMalloc(void** p, size_t n, unsigned) {
 int hipHostFree(void* p) { return drop(p); }
 int hipMemcpy(void* d, const void* s, size_t n, int) { memcpy(d, s, n); return 0; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*) {
-  if (d >= pin_lo && d < pin_hi) pinned_copies++;
   memcpy(d, s, n);
   return 0;
 }
