@@ -232,3 +232,37 @@ def test_mixed_contact_integration_in_the_acceleration_pass(wflib, n):
             assert np.abs(runs[-1]["contforce"]).sum() > 0
     for k in runs[0]:
         assert np.array_equal(runs[0][k], runs[1][k]), k
+
+
+@pytest.mark.parametrize("precision", [_abi.WF_FP64, _abi.WF_MIXED])
+@pytest.mark.parametrize("field", ["G", "rho0", "Cs", "m", "h"])
+@pytest.mark.parametrize("n,odd", [(65535, 65534), (65536, 0), (65536, 65535), (70001, 70000)])
+def test_one_value_apart_in_large_domains(oracle, wflib, n, odd, field, precision):
+    """From 65,536 values on the device finds out whether a field has one
+    value: a particle apart at either end, and uniform values again after it."""
+    sc = _scenario(n, precision, False)
+    uniform = sc.fields[field].copy()
+    st = to_oracle(oracle, sc)
+    apart = uniform.copy()
+    apart[odd] *= 1.01 if field != "h" else 1.0 + 1e-4
+    st[field] = apart
+    st.nsearch(sc.cfg)
+    st.step(sc.cfg, sc.bcs, 1)
+    with to_gpu(sc, wflib) as d:
+        d.set(field, apart)
+        d.step(1)
+        for k in MECH_FIELDS:
+            if np.linalg.norm(st[k]) > 0.0:
+                assert rel_l2(d.get(k), st[k]) <= TOL[precision], k
+        near = np.argsort(((sc.fields["x"] - sc.fields["x"][odd]) ** 2).sum(1))[:30]
+        for k in ("v", "sigma", "rho"):  # where the particle apart shows
+            assert rel_l2(d.get(k)[near], st[k][near]) <= TOL[precision], k
+    runs = []
+    for values in ([uniform], [apart, uniform]):
+        with to_gpu(sc, wflib) as d:
+            for v in values:
+                d.set(field, v)
+            d.step(2)
+            runs.append({k: d.get(k) for k in FIELDS})
+    for k in FIELDS:
+        assert np.array_equal(runs[0][k], runs[1][k]), k

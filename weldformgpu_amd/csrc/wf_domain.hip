@@ -69,6 +69,7 @@ struct wf_domain {
   char* bounce = nullptr;
   hipEvent_t bounce_ev[2 * kCopyThreads] = {};
   int device = 0;
+  int* differs = nullptr;  // a field's values differ (wf_set_field)
   int download(void* host, size_t bytes);
   Counters* ctr = nullptr;
   Counters* ctr_host = nullptr;  // pinned
@@ -381,6 +382,11 @@ __global__ void k_fill_f32v(float* a, float v, int n) {
 __global__ void k_download_i32(const int* plane, int* stage, const int* perm, int n) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s < n) stage[perm[s]] = plane[s];
+}
+// *flag = 1 if v[0..n) holds more than one value (NaN differs from all)
+__global__ void k_differs(const double* __restrict__ v, int n, int* __restrict__ flag) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > 0 && i < n && !(v[i] == v[0])) *flag = 1;
 }
 __global__ void k_iota(int* a, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -892,6 +898,7 @@ int wf_create(const wf_config* cfg, wf_domain** out) {
     if (!rc) rc = d->dev_alloc((void**)&d->mlp_scan_part, sizeof(int) * (d->npad / 1024 + 4));
     if (!rc) rc = d->dev_alloc((void**)&d->mlp_count, sizeof(int) * 4);
   }
+  if (!rc) rc = d->dev_alloc((void**)&d->differs, sizeof(int));
   if (!rc && hipHostMalloc(&d->host_i, sizeof(int) * 16) != hipSuccess) rc = WF_E_NOMEM;
   if (!rc && hipHostMalloc(&d->host_f, sizeof(float) * 16) != hipSuccess) rc = WF_E_NOMEM;
   if (!rc) {
@@ -1040,25 +1047,28 @@ int wf_set_field(wf_domain* d, int field, const void* host, size_t bytes) {
   if (field == WF_F_NB_COUNT || field == WF_F_CONT_NB_COUNT)
     return fail(WF_E_ARG, "read-only field");
   if (field == WF_F_ID || field == WF_F_M) d->surf_init = false;
-  if (field == WF_F_H) {
-    const double* hv = (const double*)host;
-    d->uniform_h = true;
-    for (int i = 1; i < d->n && d->uniform_h; i++) d->uniform_h = hv[i] == hv[0];
+  // Whether every particle has one value: looked up behind the upload, where a
+  // host scan of 2.7 M values takes as long as their upload (0.62 -> 1.27 ms);
+  // below 65,536 values the scan is the shorter one.
+  bool* uniform = field == WF_F_H      ? &d->uniform_h
+                  : field == WF_F_M    ? &d->uniform_m
+                  : field == WF_F_CS   ? &d->uniform_cs
+                  : field == WF_F_G    ? &d->uniform_G
+                  : field == WF_F_RHO0 ? &d->uniform_rho0
+                                       : nullptr;
+  const bool scan = uniform && d->n < 65536;
+  if (uniform) {
+    *uniform = false;  // until it is known
+    d->pick_arec64();
   }
-  // whether every particle has one value, and which
-  auto uniform = [&](bool& on, double& value) {
-    const double* v = (const double*)host;
-    on = true;
-    value = v[0];
-    for (int i = 1; i < d->n && on; i++) on = v[i] == v[0];
-  };
-  if (field == WF_F_M) uniform(d->uniform_m, d->m_value);
-  if (field == WF_F_CS) uniform(d->uniform_cs, d->cs_value);
-  if (field == WF_F_G) uniform(d->uniform_G, d->G_value);
-  if (field == WF_F_RHO0) uniform(d->uniform_rho0, d->rho0_value);
-  d->pick_arec64();
   if (field == WF_F_CONTFORCE || field == WF_F_Q_FRICTION) d->cf_set = true;
   HIPC(hipMemcpyAsync(d->stage, host, bytes, hipMemcpyHostToDevice, d->stream));
+  if (uniform && !scan) {
+    hipLaunchKernelGGL(k_fill_i32v, dim3(1), dim3(64), 0, d->stream, d->differs, 0, 1);
+    hipLaunchKernelGGL(k_differs, dim3(gridn(d->n)), dim3(256), 0, d->stream,
+                       (const double*)d->stage, d->n, d->differs);
+    HIPC(hipMemcpyAsync(d->host_i, d->differs, sizeof(int), hipMemcpyDeviceToHost, d->stream));
+  }
   if (elem == 8 && d->plane(field, 0).f) {
     Planes6f planes{};
     for (int c = 0; c < comps; c++) planes.p[c] = *d->plane(field, c).f;
@@ -1097,6 +1107,17 @@ int wf_set_field(wf_domain* d, int field, const void* host, size_t bytes) {
   d->mirror_dirty = true;
   HIPC(hipGetLastError());
   HIPC(hipStreamSynchronize(d->stream));
+  if (uniform) {
+    const double* v = (const double*)host;
+    bool same = scan || d->host_i[0] == 0;
+    for (int i = 1; scan && i < d->n && same; i++) same = v[i] == v[0];
+    if (field == WF_F_M) d->m_value = v[0];
+    if (field == WF_F_CS) d->cs_value = v[0];
+    if (field == WF_F_G) d->G_value = v[0];
+    if (field == WF_F_RHO0) d->rho0_value = v[0];
+    *uniform = same;
+    d->pick_arec64();
+  }
   return WF_OK;
 }
 
