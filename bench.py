@@ -56,20 +56,60 @@ sys.path.insert(0, ROOT)
 
 METRIC = "particle-updates/s: mixed+surrogate vs plain FP64 @ stated error; HBM % peak"
 HBM_PEAK_GBS = 8000.0
-# algorithmic bytes per particle-update of each kernel (FP64 plain path):
-# compulsory SoA reads + writes, neighbour data counted once, list excluded
-ALG_BYTES_FP64 = {"dens": 80, "rates": 144, "stress": 384, "accel": 144, "integrate": 172,
-                  "thermal": 120, "cond_dens": 200,
-                  # the acceleration pass integrating its particles: both
-                  # kernels' bytes less the acceleration's read back (24 B)
-                  "accel_integrate": 144 + 172 - 24,
-                  # the rates pass updating the stress: the rates are not read back
-                  "rates_stress": 144 + 384 - 72}
-# mixed (FP32 pair-loop inputs and outputs), same accounting
-ALG_BYTES_MIXED = {"dens": 40, "rates": 72, "stress": 204, "accel": 72, "integrate": 184,
-                   "thermal": 60, "cond_dens": 100, "accel_integrate": 72 + 184 - 12,
-                   "rates_stress": 72 + 204 - 36}
 
+
+def alg_bytes(mixed, surface, kept):
+    """Algorithmic bytes per particle-update of each kernel: every quantity it
+    consumes read once and every one it produces written once, at its stored
+    width (mixed precision: what the pair loops read of a particle in FP32),
+    neighbour lists, packed copies and training samples not counted.  The
+    workloads have one h, mass, sound speed, shear modulus and rest density,
+    so the last three and the stress pass's mass are arguments.
+
+    kept: the share of the steps that also store what only a caller reads
+    (wf_step: a call's last step and those that may end it); surface: the
+    rates pass takes the free-surface sums along and writes the normals."""
+    p = 4 if mixed else 8          # width in the pair loops and of the stress state
+    vec, ten = 3 * p, 6 * p
+    x = v = u = a = 24             # FP64 in both precisions
+    rho = m = h = T = sy = ep = e = q = cp = Ta = 8
+    strain, ID, BC = 48, 4, 4
+    own = rho + m if mixed else 0  # FP64 beside the pair loops' m/rho
+    near = 2 * vec + p + p         # x, v, m/rho (FP64: m; rho apart), h
+    near += 0 if mixed else rho
+    dens = (near + own + rho, rho)
+    rates = (near + 9 * p, 0)
+    if surface:
+        rates = (rates[0] + 24, 0)
+    state = rho + T + sy + ep + strain + ten + e         # read, without the rates
+    put = ten + strain + sy + ep + q + e + ten           # s, ..., sigma as the next pass reads it
+    stress = (9 * p + state + put, 3 * 8 + ten)          # kept: p, rate, sigma_eq, sigma
+    rates_stress = (rates[0] - 9 * p + state - (0 if mixed else rho) + put, stress[1] + 9 * p)
+    near_a = 2 * vec + ten + p + p + p + (p if mixed else 0)  # x, v, sigma, rho, Cs, h (FP32: m)
+    mirror = 2 * vec if mixed else 0                     # the FP32 x and v of the next passes
+    accel = (near_a + a, 0)
+    integrate = (a + x + v + u + ID + x + v + u + mirror, 0)
+    both = near_a + u + ID + (x + v if mixed else 0) + x + v + u + mirror
+    cond_r = vec + 4 * p + cp + 2 * q + Ta + BC + (T + rho if mixed else rho)  # x, T, k, m/rho, h
+    thermal = (cond_r + T + Ta + (p if mixed else 0), 16)
+    cond_dens = (cond_r + vec + (m if mixed else 0) + T + Ta + rho + (2 * p if mixed else 0), 24)
+    table = {"dens": (dens[0], 8), "rates": rates, "stress": stress, "accel": accel,
+             "integrate": integrate, "thermal": thermal, "cond_dens": cond_dens,
+             "accel_integrate": (both, 24), "rates_stress": rates_stress}
+    return {k: b + kept * extra for k, (b, extra) in table.items()}
+
+
+def kept_share(cfg, first, steps):
+    """Share of the steps first .. first + steps - 1, one wf_step call, that
+    store what only a caller reads."""
+    if cfg.rebuild_policy != 0:
+        return 1.0
+    n = cfg.ns_interval
+    moving = not cfg.quirks & 4    # rebuilds from the current snapshot
+    def kept(s):
+        return (s == first + steps - 1 or (cfg.contact and s % n == 0) or
+                ((s + 1) % n == 0 and (cfg.contact or moving)))
+    return sum(map(kept, range(first, first + steps))) / steps
 
 def _cpu_info():
     """Host CPU: model name, logical CPUs visible, physical cores (from
@@ -137,14 +177,15 @@ def cpu_baseline(sc, warm=5, steps=20, warm1=1, steps1=2):
 def profiled_traffic(workload, kernel_id):
     """HBM bytes per launch of a kernel from the committed rocprofv3 summary of
     this workload (FETCH_SIZE + WRITE_SIZE, each scaled by what the counter
-    reads for a copy kernel of known size), or None when there is none."""
+    reads for a copy kernel of known size) and the kernel profiled, or None
+    when there is none."""
     path = os.path.join(ROOT, "profiles", f"{workload}_jc_step_kernels_traffic.json")
     try:
         with open(path) as fh:
             k = json.load(fh)["kernels"].get(kernel_id)
     except (OSError, ValueError, KeyError):
-        return None
-    return None if k is None else k["fetch_bytes"] + k["write_bytes"]
+        return None, None
+    return (None, None) if k is None else (k["fetch_bytes"] + k["write_bytes"], k["kernel"])
 
 
 def workload_text(sc, n):
@@ -284,12 +325,14 @@ def main():
             dom.set_timing(True)
             dom.step(timing_steps)
             kern = {}
-            alg = ALG_BYTES_FP64 if precision == _abi.WF_FP64 else ALG_BYTES_MIXED
+            alg = alg_bytes(precision == _abi.WF_MIXED, bool(sc.cfg.contact),
+                            kept_share(sc.cfg, start + K, timing_steps))
             for k, b in alg.items():
                 ms, cnt = dom.kernel_time(k)
                 if cnt:
                     avg = ms / cnt
                     kern[k] = {"avg_ms": avg, "launches": cnt, "alg_bytes": b * sc.n,
+                               "alg_bytes_per_particle": b,
                                "GBs": b * sc.n / (avg * 1e-3) / 1e9}
             for k in ("return", "mlp", "nsearch", "contact"):
                 ms, cnt = dom.kernel_time(k)
@@ -360,15 +403,16 @@ def main():
         floor = field_err(run(_abi.WF_FP64, 0, noise=1e-12))
     kern = rmx["kern"]
     stats = rmx["s1"]
-    dom_k = max((k for k in kern if k in ALG_BYTES_MIXED), key=lambda k: kern[k]["avg_ms"])
+    dom_k = max((k for k in kern if "alg_bytes" in kern[k]), key=lambda k: kern[k]["avg_ms"])
     dk = kern[dom_k]
     # the dominant kernel's average launch in the timed steps
     avg_ms = dk["avg_ms"]
     achieved = dk["alg_bytes"] / (avg_ms * 1e-3) / 1e9
+    traffic, traffic_kernel = profiled_traffic(args.workload, "mixed/" + dom_k)
     roof = {"kernel": dom_k, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-            "traffic": profiled_traffic(args.workload, "mixed/" + dom_k),
-            "alg_bytes_per_particle": ALG_BYTES_MIXED[dom_k], "avg_ms": avg_ms,
+            "traffic": traffic, "traffic_kernel": traffic_kernel,
+            "alg_bytes_per_particle": dk["alg_bytes_per_particle"], "avg_ms": avg_ms,
             "avg_ms_back_to_back": dk.get("avg_ms_back_to_back")}
 
     cpu = None
