@@ -339,10 +339,20 @@ int wf_get_stats(struct wf_domain* d, wf_stats* out);
 /* ---- per-kernel timing with HIP events on the handle's stream ----------- */
 /* Enable (1) / disable (0) event timing; resets the accumulators.           */
 int wf_set_timing(struct wf_domain* d, int on);
-/* Kernel ids for wf_kernel_time. */
+/* Kernel ids for wf_kernel_time.  Ids are only ever added at the end, which
+ * leaves WF_ABI_VERSION (the version of the structures) as it is.  A pass of a
+ * wf_step reports under one id: where it runs inside another pass, under that
+ * one's, and its own id counts no launch.  The rates pass updates the stress
+ * (WF_K_RATES_STRESS instead of WF_K_RATES and WF_K_STRESS) where every
+ * particle has the same h, under the Johnson-Cook Newton return map only with
+ * 8,193 to 98,304 solid particles; the acceleration pass integrates
+ * (WF_K_ACCEL_INTEGRATE instead of WF_K_ACCEL and WF_K_INTEGRATE) where
+ * wf_config.fuse_integrate says; conduction takes the next step's density
+ * along (WF_K_COND_DENS instead of WF_K_THERMAL and WF_K_DENS). */
 enum {
   WF_K_DENS = 0,    /* density-rate pair loop + density update      */
-  WF_K_RATES,       /* strain/rotation-rate pair loop               */
+  WF_K_RATES,       /* strain/rotation-rate pair loop; in contact steps
+                       with one h and mass also the free-surface sums */
   WF_K_STRESS,      /* pressure + stress/plasticity + energy, with the
                        Newton Johnson-Cook return map and its
                        surrogate guess solved in place              */
@@ -353,7 +363,10 @@ enum {
   WF_K_MLP,         /* surrogate training                           */
   WF_K_RETURN,      /* reserved: the return map runs inside
                        WF_K_STRESS, so this id reports no launches  */
-  WF_K_CONTACT,     /* surface, contact neighbours, forces, mesh move */
+  WF_K_CONTACT,     /* contact steps: forces (and the integration of the
+                       particles with candidates), mesh move, each an
+                       interval a step; candidates and, where the rates
+                       pass does not sum it, the surface: one more    */
   WF_K_COND_DENS,   /* conduction pair loop + leapfrog fused with the
                        next step's density pass + update (inside one
                        wf_step call, when no rebuild runs between)  */

@@ -204,8 +204,9 @@ struct wf_domain {
   int tev_k[kTimerPool] = {0};
   int tev_n = 0;
   bool tev_pass = false;
-  // before yield: the step's max eps_p, copied to ctr_host behind the stress
-  // pass and read when the step's later passes are queued
+  // before yield: the max eps_p, copied to ctr_host behind the acceleration
+  // pass of the steps that yield_asked() names and read when the step's later
+  // passes are queued
   hipEvent_t ev_yield = nullptr;
   bool yield_pending = false;
   // yielding, under the plastic-zone trigger: the step's largest squared hot
